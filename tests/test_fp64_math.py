@@ -1,0 +1,79 @@
+"""The FP64 exp, log and reciprocal of the z-node arithmetic (threepoint_amd/csrc/tp_fp64.h), built by the host
+compiler, against 80-bit arithmetic.  The bounds follow from the forms: exp is a degree-11 polynomial whose last
+step rounds once at 0.5 ulp over an argument reduction good to 2^-56 and inner steps weighted by |r| < 0.35
+(< 1 ulp together); log adds two roundings below 0.5 ulp of the sum each and a weighted one (< 1.5 ulp); the reciprocal's third-order step
+leaves its cubed seed error and one rounding (< 1 ulp)."""
+import os
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+SRC = r"""
+#include "tp_fp64.h"
+#include <cstdio>
+#include <cmath>
+extern "C" void run(int what, int n, const double *x, double *y, long double *ref)
+{
+    for (int i = 0; i < n; ++i) {
+        if (what == 0) { y[i] = tp_fp64_exp(x[i]); if (ref) ref[i] = expl(x[i]); }
+        else if (what == 1) { y[i] = tp_fp64_log(x[i]); if (ref) ref[i] = logl(x[i]); }
+        else { y[i] = tp_fp64_rcp(x[i]); if (ref) ref[i] = 1.0L / x[i]; }
+    }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def fp64(tmp_path_factory):
+    import ctypes
+    cxx = shutil.which("g++")
+    if cxx is None:
+        pytest.skip("no host compiler")
+    d = tmp_path_factory.mktemp("fp64")
+    (d / "t.cpp").write_text(SRC)
+    subprocess.run([cxx, "-O2", "-std=c++17", "-shared", "-fPIC", "-ffp-contract=off",
+                    "-I" + os.path.join(ROOT, "threepoint_amd", "csrc"), str(d / "t.cpp"), "-o", str(d / "t.so")],
+                   check=True)
+    lib = ctypes.CDLL(str(d / "t.so"))
+
+    def call(what, x):
+        x = np.ascontiguousarray(x, dtype=np.float64)
+        y, ref = np.zeros(x.size), np.zeros(x.size, dtype=np.longdouble)
+        lib.run(what, x.size, x.ctypes.data_as(ctypes.c_void_p), y.ctypes.data_as(ctypes.c_void_p),
+                ref.ctypes.data_as(ctypes.c_void_p))
+        return y, ref
+    return call
+
+
+def _ulps(y, ref):
+    return np.max(np.abs(y.astype(np.longdouble) - ref) / np.spacing(np.abs(ref).astype(np.float64)))
+
+
+@pytest.mark.parametrize("what, bound", [(0, 1.0), (1, 1.5), (2, 1.0)])
+def test_errors(fp64, what, bound):
+    rng = np.random.default_rng(11 + what)
+    if what == 0:  # every scale down to 0, and the whole range of normal results
+        x = np.concatenate([rng.uniform(-700, 700, 200000), rng.uniform(-40, 40, 200000),
+                            rng.choice([-1, 1], 100000) * np.exp(rng.uniform(-40, 3, 100000)),
+                            np.arange(-1000, 1001) * (0.5 * np.log(2.0))])
+        x = x[np.abs(x) < 700]
+    elif what == 1:  # all binades, and both sides of 1 and of the split at sqrt(1/2)
+        x = np.concatenate([np.exp(rng.uniform(-700, 700, 200000)), 1 + rng.uniform(-1, 1, 200000) * 0.5,
+                            np.sqrt(0.5) * (1 + rng.uniform(-1, 1, 50000) * 1e-6), np.exp(rng.uniform(1, 12, 200000)),
+                            [np.finfo(float).tiny, np.finfo(float).max, 5e-324, 0.5, 2.0]])
+    else:
+        x = rng.choice([-1, 1], 400000) * np.exp(rng.uniform(-700, 700, 400000))
+    y, ref = fp64(what, x)
+    u = _ulps(y, ref)
+    print("what %d: max error %.3f ulp of %d" % (what, u, x.size))
+    assert u < bound
+
+
+def test_ends_of_the_range(fp64):
+    y, _ = fp64(0, [800.0, 5000.0, -800.0, -5000.0, 0.0, np.nan])
+    assert np.all(np.isinf(y[:2])) and np.all(y[2:4] == 0) and y[4] == 1 and np.isnan(y[5])
+    y, _ = fp64(1, [1.0, np.nan])
+    assert y[0] == 0 and np.isnan(y[1])
