@@ -1,8 +1,9 @@
 """The FP64 exp, log and reciprocal of the z-node arithmetic (threepoint_amd/csrc/tp_fp64.h), built by the host
 compiler, against 80-bit arithmetic.  The bounds follow from the forms: exp is a degree-11 polynomial whose last
 step rounds once at 0.5 ulp over an argument reduction good to 2^-56 and inner steps weighted by |r| < 0.35
-(< 1 ulp together); log adds two roundings below 0.5 ulp of the sum each and a weighted one (< 1.5 ulp); the reciprocal's third-order step
-leaves its cubed seed error and one rounding (< 1 ulp)."""
+(< 1 ulp together); log adds two roundings below 0.5 ulp of the sum each and a weighted one (< 1.5 ulp); the
+reciprocal's third-order step leaves its cubed seed error and one rounding (< 1 ulp); log1p is log's sum and one
+more addition (< 2 ulp); exp10 is exp and the rounding of its remainder's product (< 1.5 ulp)."""
 import os
 import shutil
 import subprocess
@@ -20,7 +21,9 @@ extern "C" void run(int what, int n, const double *x, double *y, long double *re
     for (int i = 0; i < n; ++i) {
         if (what == 0) { y[i] = tp_fp64_exp(x[i]); if (ref) ref[i] = expl(x[i]); }
         else if (what == 1) { y[i] = tp_fp64_log(x[i]); if (ref) ref[i] = logl(x[i]); }
-        else { y[i] = tp_fp64_rcp(x[i]); if (ref) ref[i] = 1.0L / x[i]; }
+        else if (what == 2) { y[i] = tp_fp64_rcp(x[i]); if (ref) ref[i] = 1.0L / x[i]; }
+        else if (what == 3) { y[i] = tp_fp64_log1p(x[i]); if (ref) ref[i] = log1pl(x[i]); }
+        else { y[i] = tp_fp64_exp10(x[i]); if (ref) ref[i] = powl(10.0L, x[i]); }
     }
 }
 """
@@ -49,10 +52,11 @@ def fp64(tmp_path_factory):
 
 
 def _ulps(y, ref):
-    return np.max(np.abs(y.astype(np.longdouble) - ref) / np.spacing(np.abs(ref).astype(np.float64)))
+    r = np.maximum(np.abs(ref).astype(np.float64), np.finfo(float).tiny)
+    return np.max(np.abs(y.astype(np.longdouble) - ref) / np.spacing(r))
 
 
-@pytest.mark.parametrize("what, bound", [(0, 1.0), (1, 1.5), (2, 1.0)])
+@pytest.mark.parametrize("what, bound", [(0, 1.0), (1, 1.5), (2, 1.0), (3, 2.0), (4, 1.5)])
 def test_errors(fp64, what, bound):
     rng = np.random.default_rng(11 + what)
     if what == 0:  # every scale down to 0, and the whole range of normal results
@@ -64,8 +68,12 @@ def test_errors(fp64, what, bound):
         x = np.concatenate([np.exp(rng.uniform(-700, 700, 200000)), 1 + rng.uniform(-1, 1, 200000) * 0.5,
                             np.sqrt(0.5) * (1 + rng.uniform(-1, 1, 50000) * 1e-6), np.exp(rng.uniform(1, 12, 200000)),
                             [np.finfo(float).tiny, np.finfo(float).max, 5e-324, 0.5, 2.0]])
-    else:
+    elif what == 2:
         x = rng.choice([-1, 1], 400000) * np.exp(rng.uniform(-700, 700, 400000))
+    elif what == 3:
+        x = np.concatenate([np.exp(rng.uniform(-100, 100, 400000)), rng.uniform(0, 3, 100000), [0.0, 1.0, 1e-300]])
+    else:
+        x = np.concatenate([rng.uniform(-300, 300, 200000), rng.uniform(-8, 8, 200000), np.arange(-300.0, 301.0)])
     y, ref = fp64(what, x)
     u = _ulps(y, ref)
     print("what %d: max error %.3f ulp of %d" % (what, u, x.size))

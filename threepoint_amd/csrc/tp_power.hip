@@ -122,7 +122,7 @@ __device__ double covg_point(const TpCosmoConst &C, const double *T, int n_z, do
         tp_z_at<double>(T, n_z, C.zmax, z, &Z);
         const double pref = tp_limber_pref<double>(C, z, Z.g);
         TpHaloZT<double> h;
-        tp_halofit_z<double>(C, Z, z, &h);
+        tp_halofit_z<double, TpPointFn<double>>(C, Z, z, &h);
         const double lrs = log(Z.rs), k1 = l1 / Z.fK, k2 = l2 / Z.fK, k3 = l3 / Z.fK;
         tri = pow(pref, 3) * tp_halofit_k<double>(C, Z.D1, Z.rs, lrs, h, k1, log(k1)) *
               tp_halofit_k<double>(C, Z.D1, Z.rs, lrs, h, k2, log(k2)) *
@@ -258,11 +258,13 @@ __global__ void k_power_points(const TpCosmoConst *__restrict__ cc, const double
 //      of pell_nodes, so each value has the bits of a per-point evaluation;
 //   2. one thread per point: the integrand from the cached Pell, in the reference's product order;
 //   3. one thread per region: the rule (gm_rule3, the host rule's arithmetic order).
-constexpr int kT1Reg = 5;                     // regions per workgroup: 235 Pell on 256 threads
+constexpr int kT1Reg = 4;                     // regions per workgroup: 188 Pell on 192 threads (98% of the lanes;
+                                              // 5 regions fill 235 of 256, 92%)
+constexpr int kT1Block = 192;
 constexpr int kT1Pell = 14 + TP_NPTS_GM3;     // Pell per region
 
 template <bool F32>  // F32: the Pell from the FP32 node records (pell_nodes32)
-__global__ void __launch_bounds__(256) k_t1_regions(const TpCosmoConst *__restrict__ cc,
+__global__ void __launch_bounds__(kT1Block) k_t1_regions(const TpCosmoConst *__restrict__ cc,
                                                     const TpPNode *__restrict__ pnode,
                                                     const TpPNode32 *__restrict__ pnode32, double dx,
                                                     const TpPowerDesc *__restrict__ desc,
@@ -887,7 +889,7 @@ int t1_regions(tp_ctx *ctx, const tp_cosmo *c, const std::vector<TpPowerDesc> &d
         const size_t nblk = (nreg + kT1Reg - 1) / kT1Reg;
         if (nblk > 0x7fffffffu) return tp_set_error(TP_ECAPACITY, "T1: too many regions for one launch");
         hipLaunchKernelGGL(mode == TP_MODE_FP32 ? k_t1_regions<true> : k_t1_regions<false>, dim3((unsigned)nblk),
-                           dim3(256), 0, st, c->d_const, (const TpPNode *)c->d_pnode,
+                           dim3(kT1Block), 0, st, c->d_const, (const TpPNode *)c->d_pnode,
                            (const TpPNode32 *)c->d_pnode32, c->z_max / 2, (const TpPowerDesc *)ctx->d_desc.p, d_reg,
                            nreg, d_out);
         TP_HIP(hipGetLastError());

@@ -7,6 +7,27 @@
 
 __host__ __device__ __forceinline__ double tp_dbl(double x) { return x; }
 
+// The functions of the point and node values: the library's (found by argument-dependent lookup for a counting
+// type), and for FP64 points the short forms of tp_fp64.h.  The node records of a table build keep the library's.
+struct TpLibFn {
+    template <class T> static __host__ __device__ __forceinline__ T ex(T x) { return exp(x); }
+    template <class T> static __host__ __device__ __forceinline__ T ex10(T x) { return pow(10.0, x); }
+    template <class T> static __host__ __device__ __forceinline__ T lg(T x) { return log(x); }
+    template <class T> static __host__ __device__ __forceinline__ T pw(T x, double c) { return pow(x, c); }
+};
+struct TpFastFn {
+    static __host__ __device__ __forceinline__ double ex(double x) { return tp_fp64_exp(x); }
+    static __host__ __device__ __forceinline__ double ex10(double x) { return tp_fp64_exp10(x); }
+    static __host__ __device__ __forceinline__ double lg(double x) { return tp_fp64_log(x); }
+    // powers of Omega_m(z) with |c| < 0.15: |c ln x| < 1, so the rounding of the exponent stays below an ulp of 1
+    static __host__ __device__ __forceinline__ double pw(double x, double c)
+    {
+        return x > 0 ? tp_fp64_exp(c * tp_fp64_log(x)) : __builtin_nan("");
+    }
+};
+template <class T>
+using TpPointFn = typename std::conditional<std::is_same<T, double>::value, TpFastFn, TpLibFn>::type;
+
 // Table values at redshift z (classed_version/bispectrum.cpp:506-513 + compute_coefficients :914-920).
 template <class T>
 struct TpZAtT {
@@ -46,7 +67,7 @@ struct TpHaloZT {
     T lf3c;  // ln(f3 c): the k-part takes (f3 c y)^(3 - gam) as exp((3 - gam)(ln(f3 c) + ln y))
 };
 
-template <class T>
+template <class T, class F>
 __host__ __device__ void tp_halofit_z(const TpCosmoConst &C, const TpZAtT<T> &Z, T z, TpHaloZT<T> *h)
 {
     const T n_eff = Z.ne, nsqr = n_eff * n_eff, nc = Z.nc;
@@ -55,22 +76,22 @@ __host__ __device__ void tp_halofit_z(const TpCosmoConst &C, const TpZAtT<T> &Z,
     const T den = C.om + aa * (aa * aa * C.ow + (1 - C.om - C.ow));
     const T om_m = C.om / den;
     const T om_v = C.ow * (aa * aa * aa) / den;
-    const T f1a = pow(om_m, -0.0732), f2a = pow(om_m, -0.1423), f3a = pow(om_m, 0.0725);
-    const T f1b = pow(om_m, -0.0307), f2b = pow(om_m, -0.0585), f3b = pow(om_m, 0.0743);
+    const T f1a = F::pw(om_m, -0.0732), f2a = F::pw(om_m, -0.1423), f3a = F::pw(om_m, 0.0725);
+    const T f1b = F::pw(om_m, -0.0307), f2b = F::pw(om_m, -0.0585), f3b = F::pw(om_m, 0.0743);
     const T frac = om_v / (1. - om_m);
     h->f1 = frac * f1b + (1 - frac) * f1a;
     h->f2 = frac * f2b + (1 - frac) * f2a;
     h->f3 = frac * f3b + (1 - frac) * f3a;
     T a = 1.5222 + 2.8553 * n_eff + 2.3706 * nsqr + 0.9903 * n_eff * nsqr + 0.2250 * nsqr * nsqr - 0.6038 * nc +
           0.1749 * om_v * (1.0 + C.w);
-    h->a = pow(10.0, a);
-    h->b = pow(10.0, -0.5642 + 0.5864 * n_eff + 0.5716 * nsqr - 1.5474 * nc + 0.2279 * om_v * (1.0 + C.w));
-    h->c = pow(10.0, 0.3698 + 2.0404 * n_eff + 0.8161 * nsqr + 0.5869 * nc);
+    h->a = F::ex10(a);
+    h->b = F::ex10(T(-0.5642 + 0.5864 * n_eff + 0.5716 * nsqr - 1.5474 * nc + 0.2279 * om_v * (1.0 + C.w)));
+    h->c = F::ex10(T(0.3698 + 2.0404 * n_eff + 0.8161 * nsqr + 0.5869 * nc));
     h->gam = 0.1971 - 0.0843 * n_eff + 0.8460 * nc;
     h->alpha = fabs(6.0835 + 1.3373 * n_eff - 0.1959 * nsqr - 5.5274 * nc);
     h->beta = 2.0379 - 0.7354 * n_eff + 0.3157 * nsqr + 1.2490 * n_eff * nsqr + 0.3980 * nsqr * nsqr - 0.1682 * nc;
-    h->xnu = pow(10.0, 5.2105 + 3.6902 * n_eff);
-    h->lf3c = log(h->f3 * h->c);
+    h->xnu = F::ex10(T(5.2105 + 3.6902 * n_eff));
+    h->lf3c = F::lg(T(h->f3 * h->c));
 }
 
 // The k-dependent part in log space: every power of k is exp(e ln k), with ln k supplied by the caller
@@ -97,14 +118,55 @@ __host__ __device__ T tp_pk_eh_log(const TpCosmoConst &C, T k, T lk, double norm
 template <class T>
 __host__ __device__ __forceinline__ T tp_pk_lin_log(const TpCosmoConst &C, T k, T lk)
 {
-    if constexpr (std::is_same<T, double>::value)
+    if constexpr (std::is_same<T, double>::value) {
         if (C.tab.nk) return tp_pk_table(C.tab, k);
+        return 2 * tpd::kPi * tpd::kPi * tp_delta2_lin(C, 1.0, k, lk) * tp_fp64_rcp(k * k * k);
+    }
     return tp_pk_eh_log<T>(C, k, lk, C.norm);
+}
+
+// r(k)^2 of the Eisenstein & Hu fit at kh = k h, FP64, one reciprocal per quotient pair:
+//   q_eff = kh theta^2 d / (om h^2 (sqrt(alpha_nu) d + 1 - sqrt(alpha_nu))),  d = 1 + x^4
+//   r = L / (L + (14.4 + 325 / e) q^2) = L e / (L e + (14.4 e + 325) q^2),  e = 1 + 60.5 q^1.11
+__host__ __device__ __forceinline__ double tp_eh_r2(const TpCosmoConst &C, double kh)
+{
+    const double x = 0.43 * kh * C.eh_sh, x2 = x * x, d = 1.0 + x2 * x2;
+    const double q = kh * C.eh_theta2 * d * tp_fp64_rcp(C.eh_omh2 * (C.eh_sqrt_alnu * d + (1.0 - C.eh_sqrt_alnu)));
+    const double L = tp_fp64_log(2.718281828 + C.eh_cL * q);
+    const double e = 1.0 + 60.5 * tp_fp64_exp(1.11 * tp_fp64_log(q)), Le = L * e;
+    const double r = Le * tp_fp64_rcp(Le + (14.4 * e + 325.0) * q * q);
+    return r * r;
+}
+
+// Linear Delta^2(k) = D1^2 P_lin k^3 / (2 pi^2) in FP64: the fit gives it without the k^3 it would be divided by
+__host__ __device__ __forceinline__ double tp_delta2_lin(const TpCosmoConst &C, double D1, double k, double lk)
+{
+    const double ln29979 = 8.005667322535853;  // ln 2997.9
+    if (C.tab.nk) return tp_pk_table(C.tab, k) * D1 * D1 * k * k * k / (2 * tpd::kPi * tpd::kPi);
+    const double dn = D1 * C.norm;
+    return dn * dn * tp_fp64_exp((3. + C.ns) * (lk + ln29979)) * tp_eh_r2(C, k * C.h);
+}
+
+// tp_halofit_k below in FP64 with its quotients merged to one reciprocal per term
+__host__ __device__ __forceinline__ double tp_halofit_k64(const TpCosmoConst &C, double D1, double rs, double lrs,
+                                                          const TpHaloZT<double> &h, double k, double lk)
+{
+    const double plin = tp_delta2_lin(C, D1, k, lk);
+    const double y = k * rs, ly = lk + lrs, ysqr = y * y;
+    const double den = 1 + h.b * tp_fp64_exp(h.f2 * ly) + tp_fp64_exp((3 - h.gam) * (h.lf3c + ly));
+    const double ph = h.a * tp_fp64_exp(h.f1 * 3 * ly) * ysqr * tp_fp64_rcp(den * (ysqr + h.xnu));
+    // the damping's argument is the one that leaves the range of the short exp (y up to any ell rs / f_K)
+    const double damp = tp_fp64_exp(fmax(-y * 0.25 - ysqr * 0.125, -1000.0));
+    // (a given P(k) may be negative: the library's log1p keeps its NaN below -1)
+    const double l1p = C.tab.nk ? log1p(plin) : tp_fp64_log1p(plin);
+    const double pq = plin * tp_fp64_exp(h.beta * l1p) * damp * tp_fp64_rcp(1 + plin * h.alpha);
+    return 2 * tpd::kPi * tpd::kPi * (pq + ph) * tp_fp64_rcp(k * k * k);
 }
 
 template <class T>
 __host__ __device__ T tp_halofit_k(const TpCosmoConst &C, T D1, T rs, T lrs, const TpHaloZT<T> &h, T k, T lk)
 {
+    if constexpr (std::is_same<T, double>::value) return tp_halofit_k64(C, D1, rs, lrs, h, k, lk);
     const double twopi2 = 2 * tpd::kPi * tpd::kPi;
     const T plin = tp_pk_lin_log<T>(C, k, lk) * D1 * D1 * k * k * k / twopi2;
     const T y = k * rs, ly = lk + lrs, ysqr = y * y;
@@ -118,7 +180,7 @@ template <class T>
 __host__ __device__ T tp_pnl(const TpCosmoConst &C, const TpZAtT<T> &Z, T k, T z)
 {
     TpHaloZT<T> h;
-    tp_halofit_z<T>(C, Z, z, &h);
+    tp_halofit_z<T, TpPointFn<T>>(C, Z, z, &h);
     return tp_halofit_k<T>(C, Z.D1, Z.rs, log(Z.rs), h, k, log(k));
 }
 
@@ -135,6 +197,9 @@ template <class T>
 __host__ __device__ __forceinline__ T tp_t17_factor(T lk)
 {
     const double c1 = 9.5171e-4, c2 = 5.1543e-3, a1 = 1.3063, a2 = 1.1475, a3 = 0.62793;
+    if constexpr (std::is_same<T, double>::value)
+        return tp_fp64_exp(a1 * tp_fp64_log1p(c1 * tp_fp64_exp(-a1 * lk)) -
+                           a3 * tp_fp64_log1p(c2 * tp_fp64_exp(-a2 * lk)));
     return exp(a1 * log1p(c1 * exp(-1. * a1 * lk)) - a3 * log1p(c2 * exp(-1. * a2 * lk)));
 }
 
@@ -162,7 +227,7 @@ __host__ __device__ T tp_limber_pk(const TpCosmoConst &C, const double *Tab, int
         P = Z.D1 * Z.D1 * tp_pk_lin_log<T>(C, k, lk);
     } else {
         TpHaloZT<T> h;
-        tp_halofit_z<T>(C, Z, z, &h);
+        tp_halofit_z<T, TpPointFn<T>>(C, Z, z, &h);
         P = tp_halofit_k<T>(C, Z.D1, Z.rs, log(Z.rs), h, k, lk);
     }
     return (flags & TP_PK_T17) ? tp_t17_factor<T>(lk) * pref * P : T(1.0) * pref * P;
@@ -176,6 +241,9 @@ struct TpPNode {
     TpHaloZT<double> h;
     int zero;  // z < 1e-5: the integrand is 0 there
     int pad;
+    // folded constants of tp_limber_pk_node: 1 / f_K, ln(D1^2 norm^2) + (3 + n_s) ln 2997.9, 3 + n_s, 3 f1,
+    // 3 - gam, (3 - gam) ln(f3 c), 2 pi^2 pref
+    double ifK, ld, ns3, f1x3, gam3, gl, pref2;
 };
 
 __host__ __device__ __forceinline__ void tp_pnode_make(const TpCosmoConst &C, const double *Tab, int n_z, double z,
@@ -189,9 +257,16 @@ __host__ __device__ __forceinline__ void tp_pnode_make(const TpCosmoConst &C, co
     o->lfK = log(Z.fK);
     o->lrs = log(Z.rs);
     o->pref = tp_limber_pref<double>(C, z, Z.g);
-    tp_halofit_z<double>(C, Z, z, &o->h);
+    tp_halofit_z<double, TpLibFn>(C, Z, z, &o->h);
     o->zero = z < 1e-5 ? 1 : 0;
     o->pad = 0;
+    o->ifK = 1.0 / Z.fK;
+    o->ld = log(Z.D1 * Z.D1 * C.norm * C.norm) + (3. + C.ns) * 8.005667322535853;  // ln 2997.9
+    o->ns3 = 3. + C.ns;
+    o->f1x3 = 3 * o->h.f1;
+    o->gam3 = 3 - o->h.gam;
+    o->gl = o->gam3 * o->h.lf3c;
+    o->pref2 = 2 * tpd::kPi * tpd::kPi * o->pref;
 }
 
 // FP32 form of a node record, for the FP32 Pell of T1: the node's constants folded so that a node value
@@ -267,16 +342,36 @@ __device__ __forceinline__ float tp_limber_pk_node32(const TpPNode32 &N, float e
     return v;
 }
 
-// tp_limber_pk at a precomputed node
-// (lell = ln ell, computed once per multipole)
+// tp_limber_pk at a precomputed node (lell = ln ell, computed once per multipole).  The sums over these nodes (Pell)
+// are all of T1's work and are bound by FP64 issue, so a node takes the fewest instructions its factors allow: the
+// node's constants folded, the quotients merged, the damping in the exponent of (1 + Delta^2)^beta, and 1 / k^3 in
+// that of the T17 factor, whose logarithms need no more than their absolute rounding.  A T1 covariance of 210 pairs,
+// one MI355X: 155 ms with the library's functions, 81 with those of tp_fp64.h, 73-75 in this form.
 __host__ __device__ __forceinline__ double tp_limber_pk_node(const TpCosmoConst &C, const TpPNode &N, double ell,
                                                              double lell, int flags)
 {
     if (N.zero) return 0.0;
-    const double k = ell / N.fK, lk = lell - N.lfK;
-    const double P = (flags & TP_PK_LINEAR) ? N.D1 * N.D1 * tp_pk_lin_log<double>(C, k, lk)
-                                            : tp_halofit_k<double>(C, N.D1, N.rs, N.lrs, N.h, k, lk);
-    return (flags & TP_PK_T17) ? tp_t17_factor<double>(lk) * N.pref * P : 1.0 * N.pref * P;
+    const double k = ell * N.ifK, lk = lell - N.lfK;
+    if (C.tab.nk) {  // a given P(k)
+        const double P = (flags & TP_PK_LINEAR) ? N.D1 * N.D1 * tp_pk_table(C.tab, k)
+                                                : tp_halofit_k64(C, N.D1, N.rs, N.lrs, N.h, k, lk);
+        return (flags & TP_PK_T17) ? tp_t17_factor<double>(lk) * N.pref * P : N.pref * P;
+    }
+    double P = tp_fp64_exp(fma(N.ns3, lk, N.ld)) * tp_eh_r2(C, k * C.h);  // Delta^2
+    if (!(flags & TP_PK_LINEAR)) {  // tp_halofit_k64 without its 2 pi^2 / k^3
+        const double y = k * N.rs, ly = lk + N.lrs, ysqr = y * y;
+        const double den = 1 + N.h.b * tp_fp64_exp(N.h.f2 * ly) + tp_fp64_exp(fma(N.gam3, ly, N.gl));
+        const double ph = N.h.a * tp_fp64_exp(N.f1x3 * ly) * ysqr * tp_fp64_rcp(den * (ysqr + N.h.xnu));
+        const double e = fmax(fma(N.h.beta, tp_fp64_log1p(P), -y * fma(0.125, y, 0.25)), -1000.0);
+        P = fma(P * tp_fp64_exp(e), tp_fp64_rcp(fma(P, N.h.alpha, 1.0)), ph);
+    }
+    if (flags & TP_PK_T17) {  // tp_t17_factor
+        const double c1 = 9.5171e-4, c2 = 5.1543e-3, a1 = 1.3063, a2 = 1.1475, a3 = 0.62793;
+        const double t = a1 * tp_fp64_log(fma(c1, tp_fp64_exp(-a1 * lk), 1.0)) -
+                         a3 * tp_fp64_log(fma(c2, tp_fp64_exp(-a2 * lk), 1.0));
+        return N.pref2 * P * tp_fp64_exp(fma(-3.0, lk, t));
+    }
+    return N.pref2 * P * tp_fp64_rcp(k * k * k);
 }
 
 // <Map^2> integrand at (ell, z) for one source bin, cuda_version/apertureStatistics.cu:29-57:
