@@ -450,3 +450,38 @@ def test_map3_c1_all_triples_match_oracle_fixture(fid_tables):
     assert np.all(v64[~nz] == 0) and np.all(v32[~nz] == 0)
     assert r64.max() < 1e-6 and np.array_equal(n64, nref)
     assert r32.max() < 1e-3
+
+
+@pytest.mark.parametrize("mode", [tp.MODE_FP64, tp.MODE_FP32, tp.MODE_ANALYTIC])
+@pytest.mark.parametrize("n", [1, 3, 4096, 4097, 32768, 32833, 131072, 200003])
+def test_point_calls_agree_at_every_size(fid_tables, mode, n):
+    """The evaluation calls split a point's nodes by the launch's size (one thread per node, 8 or 2 waves per point)
+    and a large call into overlapping chunks; the summation tree is the same, so a point's value is the same bits in
+    a call of any size.  Zero multipoles included (value 0)."""
+    rng = np.random.default_rng(n)
+    l = np.exp(rng.uniform(1.0, 9.0, (n, 2)))
+    phi = rng.uniform(0.0, np.pi, n)
+    ell = np.column_stack([l, np.sqrt(l[:, 0] ** 2 + l[:, 1] ** 2 + 2 * l[:, 0] * l[:, 1] * np.cos(phi))])
+    ell[n // 2, 1] = 0.0
+    x = np.column_stack([l, phi])
+    th = W.to_rad([2.0, 4.0, 8.0])
+    few = np.unique(np.concatenate([[0, n // 2, n - 1], rng.integers(0, n, 200)]))
+    b, f = fid_tables.bkappa(ell, 0, mode), fid_tables.map3_integrand(x, th, 0, mode)
+    assert np.array_equal(b[few], fid_tables.bkappa(ell[few], 0, mode))
+    assert np.array_equal(f[few], fid_tables.map3_integrand(x[few], th, 0, mode))
+    if mode != tp.MODE_ANALYTIC:
+        assert b[n // 2] == 0
+
+
+@pytest.mark.parametrize("n", [5, 70000, 140000])
+def test_non_finite_point_is_refused_and_leaves_no_flag(fid_tables, n):
+    """A non-finite ell ends the call with TP_ENONFINITE at any size, and the next call starts clean."""
+    x = np.tile([100.0, 200.0, 1.0], (n, 1))
+    th = W.to_rad([2.0, 4.0, 8.0])
+    bad = x.copy()
+    bad[n - 2, 0] = np.inf
+    good = fid_tables.map3_integrand(x, th)
+    for call in (lambda: fid_tables.map3_integrand(bad, th), lambda: fid_tables.bkappa(bad)):
+        with pytest.raises(tp.TpError, match="non-finite"):
+            call()
+        assert np.array_equal(fid_tables.map3_integrand(x, th), good)

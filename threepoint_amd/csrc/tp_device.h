@@ -411,17 +411,6 @@ __device__ __forceinline__ double tp_map3_end(const TpPointPre &P, int kind, dou
     return l1 * l2 * bk * tp_uhat<double>(l1 * th1) * tp_uhat<double>(l2 * th2) * tp_uhat<double>(l3 * th3);
 }
 
-template <class T>
-__device__ __forceinline__ double tp_map3_integrand(const TpNodeT<T> *__restrict__ nodes, const TpEHT<T> &E,
-                                                    double l1, double l2, double phi, double th1, double th2,
-                                                    double th3, int mode, int *flag)
-{
-    TpPointPre P;
-    const int kind = tp_map3_begin(l1, l2, phi, mode, flag, &P);
-    const double s = kind == TP_PT_SUM ? tp_bkappa_parts<T, TP_NPART>(nodes, E, P, 0) : 0.0;
-    return tp_map3_end(P, kind, s, th1, th2, th3, flag);
-}
-
 // --------------------------------------------------- Genz-Malik 3-D rule
 // Point p of a region, in the reference's order (classed_version/hcubature.cpp:
 // 343-414, 476-503): center; -+lambda2, -+lambda4 on each axis; (lambda4,lambda4)

@@ -160,6 +160,7 @@ struct TpLane {
     int create();
     void release();
 };
+constexpr int kPointsMaxChunks = 16;  // chunks of a point-evaluation call (run_points)
 constexpr int TP_NLANES = 4;  // groups of a batched call (at most; tp_ctx::nlanes are used)
 
 constexpr size_t kTpKeepPoolBytes = size_t(16) << 30;  // default cap on the host region pools kept
@@ -219,6 +220,12 @@ struct tp_ctx {
     bool round_log_on = false;        // tp_set_round_log: per-round trace of tp_map3_batch
     std::vector<double> round_log;    // 7 doubles per round (tp_round_log)
     TpLane lane[TP_NLANES];
+    // point-evaluation calls (run_points): an event per chunk, and the flag word, which is zero between calls.
+    // Created on the first such call.
+    hipEvent_t pt_out[kPointsMaxChunks] = {};
+    DevBuf d_ptflag;
+    int points_create(bool chunks);
+    void points_release();
 };
 
 // OpenMP threads for the host side of the batched cubatures (region records, heaps):
@@ -246,11 +253,11 @@ void tp_gauss_legendre(int n, double *x, double *w);
 // Builds c->d_pnode from c's tables (tp_power.hip); called at the end of every table build.
 int tp_build_pnodes(tp_ctx *ctx, tp_cosmo *c);
 
-// Launchers implemented in the .hip files (all asynchronous on ctx->stream).
-int tp_launch_map3_points(tp_ctx *ctx, const tp_cosmo *c, int icosmo, const double *th, size_t npts,
-                          const double *d_x, double *d_f, int mode, int *d_flag);
-int tp_launch_bkappa_points(tp_ctx *ctx, const tp_cosmo *c, int icosmo, size_t npts, const double *d_l,
-                            double *d_out, int mode, int *d_flag);
+// Launchers implemented in the .hip files (all asynchronous on st).
+int tp_launch_map3_points(const tp_cosmo *c, int icosmo, const double *th, size_t npts, const double *d_x, double *d_f,
+                          int mode, int *d_flag, hipStream_t st);
+int tp_launch_bkappa_points(const tp_cosmo *c, int icosmo, size_t npts, const double *d_l, double *d_out, int mode,
+                            int *d_flag, hipStream_t st);
 int tp_launch_regions(tp_ctx *ctx, const tp_cosmo *c, size_t nreg, const TpRegion *d_reg,
                       const TpIntegralDesc *d_desc, double *d_fvals, TpRegionOut *d_out, int mode,
                       int *d_flag, hipEvent_t evm, hipStream_t st);

@@ -22,35 +22,147 @@
 namespace {
 
 // --------------------------------------------------------------- kernels
-template <class T>
-__global__ void __launch_bounds__(256) k_map3_points(const TpNodeT<T> *__restrict__ nodes,
-                                                     const TpEHT<T> *__restrict__ eh, double th1, double th2,
-                                                     double th3, size_t npts, const double *__restrict__ x,
-                                                     double *__restrict__ f, int mode, int *flag)
+// Points of the evaluation calls: B_kappa at (l1, l2, l3) rows, or the <Map^3> integrand at (l1, l2, phi) rows.
+// Set-up of a point and its value from the z-sum, for the kernels below that split the sum differently.
+struct PointTh {
+    double t[3];  // aperture radii of the <Map^3> integrand
+};
+template <bool MAP3>
+__device__ __forceinline__ int point_begin(const double *__restrict__ x, size_t i, int mode, int *flag, TpPointPre *P)
 {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= npts) return;
-    double l1 = x[3 * i], l2 = x[3 * i + 1], phi = x[3 * i + 2];
-    double v = tp_map3_integrand<T>(nodes, *eh, l1, l2, phi, th1, th2, th3, mode, flag);
-    f[i] = v;
+    const double a = x[3 * i], b = x[3 * i + 1], c = x[3 * i + 2];
+    if (MAP3) return tp_map3_begin(a, b, c, mode, flag, P);
+    P->l[0] = a;
+    P->l[1] = b;
+    P->l[2] = c;
+    if (a == 0 || b == 0 || c == 0 || mode == TP_MODE_ANALYTIC) return TP_PT_NOSUM;
+    tp_point_pre<double>(a, b, c, P);
+    return TP_PT_SUM;
+}
+template <bool MAP3>
+__device__ __forceinline__ double point_end(const TpPointPre &P, int kind, double sum, const PointTh &th, int mode,
+                                            int *flag)
+{
+    if (MAP3) return tp_map3_end(P, kind, sum, th.t[0], th.t[1], th.t[2], flag);
+    double v = sum;
+    if (kind != TP_PT_SUM) v = mode == TP_MODE_ANALYTIC ? tp_bkappa_analytic(P.l[0], P.l[1], P.l[2]) : 0.0;
+    if (!isfinite(v)) atomicOr(flag, 1);
+    return v;
 }
 
-template <class T>
-__global__ void __launch_bounds__(256) k_bkappa_points(const TpNodeT<T> *__restrict__ nodes,
-                                                       const TpEHT<T> *__restrict__ eh, size_t npts,
-                                                       const double *__restrict__ l, double *__restrict__ out,
-                                                       int mode, int *flag)
+// A point's 96 nodes split over LPP waves (a power of two up to 8), the fixed summation tree of k_region_points: one thread per
+// point takes ~100 us (FP32) to ~270 us (FP64) however few the points are, since its 96 nodes are one serial chain.
+template <class T, int LPP, bool MAP3>
+__global__ void __launch_bounds__(64 * (LPP < 4 ? 4 : LPP)) k_points(const TpNodeT<T> *__restrict__ nodes,
+                                                                     const TpEHT<T> *__restrict__ eh, PointTh th,
+                                                                     size_t npts, const double *__restrict__ x,
+                                                                     double *__restrict__ f, int mode, int *flag)
 {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= npts) return;
-    double l1 = l[3 * i], l2 = l[3 * i + 1], l3 = l[3 * i + 2];
-    double v;
-    if (mode == TP_MODE_ANALYTIC)
-        v = tp_bkappa_analytic(l1, l2, l3);
-    else
-        v = (l1 == 0 || l2 == 0 || l3 == 0) ? 0.0 : tp_bkappa_sum<T>(nodes, *eh, l1, l2, l3);
-    if (!isfinite(v)) atomicOr(flag, 1);
-    out[i] = v;
+    constexpr int GPB = LPP < 4 ? 4 / LPP : 1;  // groups of 64 points per workgroup
+    __shared__ double part[GPB][LPP][64];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), g = wv / LPP,
+              w = wv % LPP;
+    const size_t i = ((size_t)blockIdx.x * GPB + g) * 64 + lane;
+    TpPointPre P;
+    int kind = TP_PT_DONE;
+    double v = 0.0;
+    if (i < npts) {
+        kind = point_begin<MAP3>(x, i, mode, flag, &P);
+        if (kind == TP_PT_SUM) v = tp_bkappa_parts<T, TP_NPART / LPP>(nodes, *eh, P, w * (TP_NPART / LPP));
+    }
+    if constexpr (LPP > 1) {
+        part[g][w][lane] = v;
+        __syncthreads();
+        if (w != 0) return;
+        double a[LPP];
+#pragma unroll
+        for (int k = 0; k < LPP; ++k) a[k] = part[g][k][lane];
+#pragma unroll
+        for (int s = 1; s < LPP; s <<= 1)
+#pragma unroll
+            for (int k = 0; k < LPP; k += 2 * s) a[k] = a[k] + a[k + s];
+        v = a[0];
+    }
+    if (i < npts) f[i] = point_end<MAP3>(P, kind, v, th, mode, flag);
+}
+
+// The fewest points: one thread per (point, node), two points per workgroup of three waves.  Every thread of a point
+// forms its set-up (no exchange, no barrier before the node), the node values go to LDS, eight threads add the
+// partials in node order and one joins the tree -- the bits of every other split.  The chain is one node instead of
+// twelve (8 waves per point); the set-up, repeated 96 times, is ~0.7 of a node's work, so it pays only while the
+// launch leaves the chip idle.
+constexpr int kNodePts = 2, kNodeBlock = kNodePts * TP_NNODES;  // 192 threads
+
+// value of node `node` for the point, into val[node]; the sum over all nodes for the threads with node == 0
+template <class T>
+__device__ __forceinline__ double node_sum(const TpNodeT<T> *__restrict__ nodes, const TpEHT<T> &E, const TpPointPre &P,
+                                           bool sum, int node, T *val, double *part)
+{
+    if (sum) {
+        const TpNodeT<T> &N = nodes[node];
+        const T ks = N.ks, lks = N.lnks;
+        const T q[3] = {(T)P.l[0] * ks, (T)P.l[1] * ks, (T)P.l[2] * ks};
+        const T lq[3] = {(T)P.ll[0] + lks, (T)P.ll[1] + lks, (T)P.ll[2] + lks};
+        const T f2t[3] = {(T)P.f2t[0], (T)P.f2t[1], (T)P.f2t[2]};
+        val[node] = tp_bispec_node<T>(N, E, q, lq, f2t, (T)P.lr1, (T)P.r2);
+    }
+    __syncthreads();
+    if (sum && node < TP_NPART) {
+        double acc = 0.0;
+        for (int j = 0; j < TP_PART_NODES; ++j) {
+            const int n = node * TP_PART_NODES + j;
+            acc += (double)(nodes[n].wz * val[n]);
+        }
+        part[node] = acc;
+    }
+    __syncthreads();
+    if (!sum || node != 0) return 0.0;
+    return ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
+}
+
+template <class T, bool MAP3>
+__global__ void __launch_bounds__(kNodeBlock) k_points_nodes(const TpNodeT<T> *__restrict__ nodes,
+                                                             const TpEHT<T> *__restrict__ eh, PointTh th, size_t npts,
+                                                             const double *__restrict__ x, double *__restrict__ f,
+                                                             int mode, int *flag)
+{
+    __shared__ T val[kNodePts][TP_NNODES];
+    __shared__ double part[kNodePts][TP_NPART];
+    const int p = threadIdx.x / TP_NNODES, node = threadIdx.x - p * TP_NNODES;
+    const size_t i = (size_t)blockIdx.x * kNodePts + p;
+    TpPointPre P;
+    const int kind = i < npts ? point_begin<MAP3>(x, i, mode, flag, &P) : TP_PT_DONE;
+    const double v = node_sum<T>(nodes, *eh, P, kind == TP_PT_SUM, node, val[p], part[p]);
+    if (i < npts && node == 0) f[i] = point_end<MAP3>(P, kind, v, th, mode, flag);
+}
+
+// The same split for the regions of a batch's smallest rounds.
+template <class T>
+__global__ void __launch_bounds__(kNodeBlock) k_region_nodes(const TpNodeT<T> *__restrict__ nodes,
+                                                             const TpEHT<T> *__restrict__ eh, size_t nreg,
+                                                             const TpRegion *__restrict__ reg,
+                                                             const TpIntegralDesc *__restrict__ desc,
+                                                             double *__restrict__ fvals, int mode, int *flag)
+{
+    __shared__ T val[kNodePts][TP_NNODES];
+    __shared__ double part[kNodePts][TP_NPART];
+    const int p = threadIdx.x / TP_NNODES, node = threadIdx.x - p * TP_NNODES;
+    const size_t t = (size_t)blockIdx.x * kNodePts + p;
+    const bool live = t < nreg * TP_NPTS_GM3;
+    TpPointPre P;
+    int kind = TP_PT_DONE;
+    TpIntegralDesc D{};
+    if (live) {
+        const size_t r = t / TP_NPTS_GM3;
+        const TpRegion R = reg[r];
+        D = desc[R.integral];
+        double x0, x1, x2;
+        gm_point3(R, (int)(t - r * TP_NPTS_GM3), &x0, &x1, &x2);
+        kind = tp_map3_begin(x0, x1, x2, mode, flag, &P);
+    }
+    const double v = node_sum<T>(nodes + (size_t)D.icosmo * TP_NNODES, eh[D.icosmo], P, kind == TP_PT_SUM, node, val[p],
+                                 part[p]);
+    if (live && node == 0) fvals[t] = tp_map3_end(P, kind, v, D.th[0], D.th[1], D.th[2], flag);
 }
 
 // Integrand values of the 33 Genz-Malik points of many regions of many integrals.  A point's 96
@@ -285,39 +397,62 @@ int grid_for(size_t n, int block) { return (int)((n + block - 1) / block); }
 
 }  // namespace
 
-int tp_launch_map3_points(tp_ctx *ctx, const tp_cosmo *c, int icosmo, const double *th, size_t npts,
+// The split of a point's nodes by launch size, from whole calls of B_kappa (us; FP64, FP32 in brackets) with one
+// thread per (point, node), 8, 2 and 1 waves per point:
+//      33 points:  21 (20)   65 (35)  133 (57)  249 (95)     4 096:  45 (36)    68 (38)  136 (62)  254 (102)
+//     8 192:       90 (68)   93 (61)  160 (84)  278 (126)   32 768: 224 (159)  170 (107) 195 (116) 307 (156)
+//    65 536:                299 (174) 310 (183) 357 (204)  131 072:            555 (326) 546 (322) 576 (335)
+// one thread per (point, node) while its repeated set-up costs less than the shorter chain gains, 8 waves until the
+// launch fills the chip with fewer, then 2.
+constexpr size_t kNodePoints = 4096, kWidePoints = 131072;
+
+template <class T, bool MAP3>
+static void launch_points(hipStream_t st, const TpNodeT<T> *nodes, const TpEHT<T> *eh, const PointTh &th, size_t npts,
                           const double *d_x, double *d_f, int mode, int *d_flag)
 {
-    if (npts == 0) return 0;
-    const int B = 256;
-    if (mode == TP_MODE_FP32)
-        hipLaunchKernelGGL(k_map3_points<float>, dim3(grid_for(npts, B)), dim3(B), 0, ctx->stream,
-                           c->d_node32 + (size_t)icosmo * TP_NNODES, c->d_eh32 + icosmo, th[0], th[1], th[2], npts,
-                           d_x, d_f, mode, d_flag);
+    const size_t groups = (npts + 63) / 64;
+    if (npts <= kNodePoints)
+        hipLaunchKernelGGL((k_points_nodes<T, MAP3>), dim3((unsigned)((npts + kNodePts - 1) / kNodePts)),
+                           dim3(kNodeBlock), 0, st, nodes, eh, th, npts, d_x, d_f, mode, d_flag);
+    else if (npts < kWidePoints)
+        hipLaunchKernelGGL((k_points<T, 8, MAP3>), dim3((unsigned)groups), dim3(512), 0, st, nodes, eh, th, npts, d_x,
+                           d_f, mode, d_flag);
     else
-        hipLaunchKernelGGL(k_map3_points<double>, dim3(grid_for(npts, B)), dim3(B), 0, ctx->stream,
-                           c->d_node64 + (size_t)icosmo * TP_NNODES, c->d_eh64 + icosmo, th[0], th[1], th[2], npts,
-                           d_x, d_f, mode, d_flag);
+        hipLaunchKernelGGL((k_points<T, 2, MAP3>), dim3((unsigned)((groups + 1) / 2)), dim3(256), 0, st, nodes, eh, th,
+                           npts, d_x, d_f, mode, d_flag);
+}
+
+template <bool MAP3>
+static int launch_points_mode(const tp_cosmo *c, int icosmo, const PointTh &th, size_t npts, const double *d_x,
+                              double *d_f, int mode, int *d_flag, hipStream_t st)
+{
+    if (npts == 0) return 0;
+    const size_t o = (size_t)icosmo * TP_NNODES;
+    if (mode == TP_MODE_FP32)
+        launch_points<float, MAP3>(st, c->d_node32 + o, c->d_eh32 + icosmo, th, npts, d_x, d_f, mode, d_flag);
+    else
+        launch_points<double, MAP3>(st, c->d_node64 + o, c->d_eh64 + icosmo, th, npts, d_x, d_f, mode, d_flag);
     TP_HIP(hipGetLastError());
     return 0;
 }
 
-int tp_launch_bkappa_points(tp_ctx *ctx, const tp_cosmo *c, int icosmo, size_t npts, const double *d_l,
-                            double *d_out, int mode, int *d_flag)
+int tp_launch_map3_points(const tp_cosmo *c, int icosmo, const double *th, size_t npts, const double *d_x, double *d_f,
+                          int mode, int *d_flag, hipStream_t st)
 {
-    if (npts == 0) return 0;
-    const int B = 256;
-    if (mode == TP_MODE_FP32)
-        hipLaunchKernelGGL(k_bkappa_points<float>, dim3(grid_for(npts, B)), dim3(B), 0, ctx->stream,
-                           c->d_node32 + (size_t)icosmo * TP_NNODES, c->d_eh32 + icosmo, npts, d_l, d_out, mode,
-                           d_flag);
-    else
-        hipLaunchKernelGGL(k_bkappa_points<double>, dim3(grid_for(npts, B)), dim3(B), 0, ctx->stream,
-                           c->d_node64 + (size_t)icosmo * TP_NNODES, c->d_eh64 + icosmo, npts, d_l, d_out, mode,
-                           d_flag);
-    TP_HIP(hipGetLastError());
-    return 0;
+    return launch_points_mode<true>(c, icosmo, PointTh{{th[0], th[1], th[2]}}, npts, d_x, d_f, mode, d_flag, st);
 }
+
+int tp_launch_bkappa_points(const tp_cosmo *c, int icosmo, size_t npts, const double *d_l, double *d_out, int mode,
+                            int *d_flag, hipStream_t st)
+{
+    return launch_points_mode<false>(c, icosmo, PointTh{}, npts, d_l, d_out, mode, d_flag, st);
+}
+
+// The launch shape of k_region_nodes, taken by rounds of up to 32 regions: those read their region records from host
+// memory, every wave its own, so the shape's many waves cost more there than in a point call (one FP32 integral:
+// 1.91 ms without it, 1.48 up to 32 regions; 220 integrals: 24.6, 24.7, and 26.5 up to 124 regions).
+constexpr int kShapeNodes = 96;
+constexpr size_t kNodeRegionPoints = 32 * TP_NPTS_GM3;
 
 // one launch of the region-point kernel with LPP waves per point group
 template <class T>
@@ -328,6 +463,10 @@ static void launch_region_points(hipStream_t st, int lpp, const TpNodeT<T> *node
     const size_t np = nreg * TP_NPTS_GM3;
     const size_t groups = (np + 63) / 64;
     switch (lpp) {
+    case kShapeNodes:
+        hipLaunchKernelGGL((k_region_nodes<T>), dim3((unsigned)((np + kNodePts - 1) / kNodePts)), dim3(kNodeBlock), 0,
+                           st, nodes, eh, nreg, d_reg, d_desc, d_fvals, mode, d_flag);
+        break;
     case 2:
         hipLaunchKernelGGL((k_region_points<T, 2>), dim3((unsigned)((groups + 1) / 2)), dim3(256), 0, st, nodes, eh,
                            nreg, d_reg, d_desc, d_fvals, mode, d_flag);
@@ -392,6 +531,11 @@ static void region_points_shape(int lpp, size_t nreg, void **func, dim3 *grid, d
 {
     const size_t groups = (nreg * TP_NPTS_GM3 + 63) / 64;
     switch (lpp) {
+    case kShapeNodes:
+        *func = (void *)k_region_nodes<T>;
+        *grid = dim3((unsigned)((nreg * TP_NPTS_GM3 + kNodePts - 1) / kNodePts));
+        *block = dim3(kNodeBlock);
+        break;
     case 2:
         *func = (void *)k_region_points<T, 2>;
         *grid = dim3((unsigned)((groups + 1) / 2));
@@ -569,7 +713,7 @@ int tp_region_lanes(tp_ctx *ctx, const tp_cosmo *c, int mode, size_t np)
         if (e1) (void)hipEventDestroy(e1);
         if (!ok) return tp_set_error(TP_EHIP, "tp_launch_regions: launch-shape tuning failed"), -1;
     }
-    return ctx->region_lpp[im][region_bucket(np)];
+    return np <= kNodeRegionPoints ? kShapeNodes : ctx->region_lpp[im][region_bucket(np)];
 }
 
 extern "C" int tp_set_region_lanes(tp_ctx *ctx, int lanes)
