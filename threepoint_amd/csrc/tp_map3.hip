@@ -220,7 +220,7 @@ __global__ void __launch_bounds__(64 * (LPP < 4 ? 4 : LPP)) k_region_points(
 // workgroup takes kCacheReg regions with G groups of 256 threads; group g owns the partials
 // [g 8/G, (g+1) 8/G) of the summation tree and, for each partial (12 z-nodes),
 //   A. evaluates the P_E terms of the 47 multipoles per region (7 l1, 7 l2, 33 l3) at the 12 nodes
-//      into its LDS block (work items of 64 consecutive (node, multipole) entries, whose at most two
+//      into its LDS block (work items of one node and 64 multipoles, and the remainders of all nodes
 //      node records are read through wave-uniform loads);
 //   B. lets each point add its 12 node values, the shape-dependent rest (tp_bispec_joint) with the
 //      three P_E terms read from LDS, and push the partial into the group's subtree.
@@ -228,12 +228,13 @@ __global__ void __launch_bounds__(64 * (LPP < 4 ? 4 : LPP)) k_region_points(
 // as in k_region_points, so every shape gives the same bits.  More groups shorten a thread's share
 // of the work, which keeps launches of a few thousand regions from ending on a half-empty wave of
 // workgroups.
-constexpr int kCacheReg = 7;                       // regions per workgroup: 231 points per group
-constexpr int kCacheEll = 14 + TP_NPTS_GM3;        // multipoles per region: 7 l1, 7 l2, 33 l3
-constexpr int kCacheN = kCacheReg * kCacheEll;     // 329
+constexpr int kCacheReg = 7, kCacheThreads = 256;  // regions per workgroup and threads per group
+constexpr int kCacheSets = 2 * kCacheReg;          // (region, axis) sets of 7 multipoles l1 or l2
+constexpr int kCacheN = 7 * kCacheSets + TP_NPTS_GM3 * kCacheReg;  // multipoles at most: 329
+static_assert(kCacheSets <= 64 && TP_NPTS_GM3 * kCacheReg <= kCacheThreads && 7 * kCacheSets <= kCacheThreads, "");
 
 template <class T, int G>
-__global__ void __launch_bounds__(256 * G) k_region_cached(const TpNodeT<T> *__restrict__ nodes,
+__global__ void __launch_bounds__(kCacheThreads * G) k_region_cached(const TpNodeT<T> *__restrict__ nodes,
                                                            const TpEHT<T> *__restrict__ eh, size_t nreg,
                                                            const TpRegion *__restrict__ reg,
                                                            const TpIntegralDesc *__restrict__ desc,
@@ -243,16 +244,48 @@ __global__ void __launch_bounds__(256 * G) k_region_cached(const TpNodeT<T> *__r
     __shared__ T lv[kCacheN], llv[kCacheN];           // multipole and its log, as the points see them
     __shared__ T pse[G][TP_PART_NODES][kCacheN];      // P_E at (group, node of the partial, multipole)
     __shared__ double sub[G > 1 ? G : 1][kCacheReg * TP_NPTS_GM3];  // the groups' subtree values
-    __shared__ int ics[kCacheReg];                    // cosmology of each region
-    __shared__ int one_cosmo;                         // all regions of the workgroup share ics[0]
-    const int t = threadIdx.x & 255, lane = t & 63;
-    const int g = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8);
+    __shared__ double set_c[kCacheSets], set_h[kCacheSets];  // centre and half width of each (region, axis) set
+    __shared__ int set_ic[kCacheSets];                // its cosmology (set 2 rr: of region rr)
+    __shared__ int slot[kCacheSets], uset[kCacheSets];  // a set's place among the distinct ones; a place's set
+    __shared__ int n_uset, one_cosmo;                 // distinct sets; all regions of the workgroup share a cosmology
+    constexpr int NW = kCacheThreads / 64;
+    const int g = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kCacheThreads);
+    const int t = threadIdx.x - g * kCacheThreads, lane = t & 63;
     const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
     const size_t r0 = (size_t)blockIdx.x * kCacheReg;
     const int nr = (int)((nreg - r0) < (size_t)kCacheReg ? (nreg - r0) : (size_t)kCacheReg);  // >= 1
-    const int ne = nr * kCacheEll;
-    // set-up: every group's point threads form their point; group 0 stores the l3 entries and
-    // its threads < 14 nr the l1 / l2 entries
+    const int ns = 2 * nr;
+    // distinct sets: wave 0 of group 0, one lane per set (lanes of one wave exchange through LDS, in order)
+    if (threadIdx.x < 64) {
+        double c = 0.0, h = 0.0;
+        int ic = 0;
+        if (lane < ns) {
+            const TpRegion &R = reg[r0 + (lane >> 1)];
+            c = R.c[lane & 1];
+            h = R.hw[lane & 1];
+            ic = desc[R.integral].icosmo;
+            set_c[lane] = c;
+            set_h[lane] = h;
+            set_ic[lane] = ic;
+        }
+        __builtin_amdgcn_wave_barrier();
+        __threadfence_block();
+        int first = lane;
+        for (int k = ns - 1; k >= 0; --k)
+            if (k < lane && lane < ns && set_c[k] == c && set_h[k] == h && set_ic[k] == ic) first = k;
+        const unsigned long long uniq = __ballot(lane < ns && first == lane);
+        if (lane < ns) {
+            const int at = __popcll(uniq & ((1ull << first) - 1));
+            slot[lane] = at;
+            if (first == lane) uset[at] = lane;
+        }
+        const unsigned long long other = __ballot(lane < ns && ic != __builtin_amdgcn_readfirstlane(ic));
+        if (lane == 0) {
+            n_uset = __popcll(uniq);
+            one_cosmo = other == 0;
+        }
+    }
+    // every group's point threads form their point
     const bool pt = t < nr * TP_NPTS_GM3;
     const int prr = t / TP_NPTS_GM3, pp = t - prr * TP_NPTS_GM3;
     TpPointPre P;
@@ -264,30 +297,28 @@ __global__ void __launch_bounds__(256 * G) k_region_cached(const TpNodeT<T> *__r
         double x0, x1, x2;
         gm_point3(R, pp, &x0, &x1, &x2);
         kind = tp_map3_begin(x0, x1, x2, mode, flag, &P);  // every group flags the same points: same bit
-        if (g == 0) {
-            const int e = prr * kCacheEll + 14 + pp;
-            lv[e] = kind == TP_PT_SUM ? (T)P.l[2] : T(1);
-            llv[e] = kind == TP_PT_SUM ? (T)P.ll[2] : T(0);
-            if (pp == 0) ics[prr] = D.icosmo;
-        }
-    }
-    if (g == 0 && t < nr * 14) {
-        const int rr = t / 14, k = t - rr * 14, ax = k / 7;  // k = 7 axis + code + 3
-        const TpRegion R = reg[r0 + rr];
-        const double x = tp_gm_coord(ax ? R.c[1] : R.c[0], ax ? R.hw[1] : R.hw[0], k - 7 * ax - 3);
-        lv[rr * kCacheEll + k] = (T)x;
-        llv[rr * kCacheEll + k] = x > 0 ? (T)TpMath<double>::lg(x) : T(0);  // non-positive: no summed point uses it
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        int u = 1;
-        for (int rr = 1; rr < nr; ++rr) u &= ics[rr] == ics[0];
-        one_cosmo = u;
+    // group 0 stores the multipoles: the distinct sets', then the points' l3
+    const int nu7 = 7 * __builtin_amdgcn_readfirstlane(n_uset);
+    const int ne = nu7 + nr * TP_NPTS_GM3;
+    if (g == 0) {
+        if (pt) {
+            const int e = nu7 + t;
+            lv[e] = kind == TP_PT_SUM ? (T)P.l[2] : T(1);
+            llv[e] = kind == TP_PT_SUM ? (T)P.ll[2] : T(0);
+        }
+        if (t < nu7) {
+            const int u = uset[t / 7];
+            const double x = tp_gm_coord(set_c[u], set_h[u], t % 7 - 3);
+            lv[t] = (T)x;
+            llv[t] = x > 0 ? (T)TpMath<double>::lg(x) : T(0);  // non-positive: no summed point uses it
+        }
     }
     __syncthreads();
     // block-uniform: with one cosmology the node and E&H records are read through scalar loads
     const int uni = __builtin_amdgcn_readfirstlane(one_cosmo);
-    const int ic0 = __builtin_amdgcn_readfirstlane(ics[0]);
+    const int ic0 = __builtin_amdgcn_readfirstlane(set_ic[0]);
     const TpNodeT<T> *__restrict__ nodes0 = nodes + (size_t)ic0 * TP_NNODES;
     const bool sum = pt && kind == TP_PT_SUM;
     T L[3] = {T(1), T(1), T(1)}, LL[3] = {T(0), T(0), T(0)}, F2T[3] = {T(0), T(0), T(0)}, LR1 = T(0), R2 = T(0);
@@ -301,10 +332,9 @@ __global__ void __launch_bounds__(256 * G) k_region_cached(const TpNodeT<T> *__r
         }
         LR1 = (T)P.lr1;
         R2 = (T)P.r2;
-        const int base = prr * kCacheEll;
-        e0 = base + c_gm3_code[pp][0] + 3;
-        e1 = base + c_gm3_code[pp][1] + 10;
-        e2 = base + 14 + pp;
+        e0 = 7 * slot[2 * prr] + c_gm3_code[pp][0] + 3;
+        e1 = 7 * slot[2 * prr + 1] + c_gm3_code[pp][1] + 3;
+        e2 = nu7 + t;
         Np = nodes + (size_t)D.icosmo * TP_NNODES;
     }
     T(*ps_g)[kCacheN] = pse[g];
@@ -322,39 +352,38 @@ __global__ void __launch_bounds__(256 * G) k_region_cached(const TpNodeT<T> *__r
         }
         return acc;
     };
-    // phase A work items.  With one cosmology and at least two regions (ne >= 94): 64 consecutive
-    // entries of the flattened (node j, multipole e) space of the partial, so that every lane has
-    // work; such an item spans at most two nodes, read as two wave-uniform records and selected per
-    // lane.  Otherwise: one node and 64 consecutive multipoles.
-    const bool flat = uni && ne >= 64;
-    const int nflat = TP_PART_NODES * ne;
-    const int nblk = (ne + 63) >> 6, items = flat ? (nflat + 63) >> 6 : TP_PART_NODES * nblk;
+    // phase A work items.  One cosmology: the full chunks of 64 multipoles, one node each (wave-uniform records, scalar
+    // loads), then the last ne % 64 multipoles of all 12 nodes packed into chunks of 64 (records per lane).  More
+    // cosmologies: one node and 64 multipoles, records per lane.
+    const int nfull = uni ? ne >> 6 : 0, tail = ne - 64 * nfull, ntail = TP_PART_NODES * tail;
+    const int nblk = (ne + 63) >> 6;
     double s1 = 0.0, s2 = 0.0, s4 = 0.0, v = 0.0;
     for (int k = 0; k < PPG; ++k) {
         const int n0 = (g * PPG + k) * TP_PART_NODES;
-        if (flat) {
-            for (int it = wv; it < items; it += 4) {
-                const int f = it * 64 + lane;
-                const int ja = (it * 64) / ne, jb = min(ja + 1, TP_PART_NODES - 1);  // wave-uniform
-                const TpNodeT<T> &Na = nodes0[n0 + ja], &Nb = nodes0[n0 + jb];
-                if (f < nflat) {
-                    const int j = f / ne, e = f - j * ne;
-                    const TpNodeT<T> N = j == ja ? Na : Nb;
-                    ps_g[j][e] = tp_pse_node<T>(N, eh[ic0], lv[e] * N.ks, llv[e] + N.lnks);
+        if (uni) {
+            int j = 0, c = wv;  // (node, chunk) of item wv, wv + NW, ...; past the last node c counts the tail's items
+            for (; nfull; c += NW) {
+                while (c >= nfull && j < TP_PART_NODES) {
+                    c -= nfull;
+                    ++j;
                 }
+                if (j >= TP_PART_NODES) break;
+                const TpNodeT<T> &N = nodes0[n0 + j];
+                const int e = c * 64 + lane;
+                ps_g[j][e] = tp_pse_node<T>(N, eh[ic0], lv[e] * N.ks, llv[e] + N.lnks);
+            }
+            for (int f = c * 64 + lane; f < ntail; f += kCacheThreads) {
+                const int jt = f / tail, e = 64 * nfull + f - jt * tail;
+                const TpNodeT<T> &N = nodes0[n0 + jt];
+                ps_g[jt][e] = tp_pse_node<T>(N, eh[ic0], lv[e] * N.ks, llv[e] + N.lnks);
             }
         } else {
-            for (int it = wv; it < items; it += 4) {
+            for (int it = wv; it < TP_PART_NODES * nblk; it += NW) {
                 const int j = it / nblk, e = (it - j * nblk) * 64 + lane;
                 if (e < ne) {
-                    if (uni) {
-                        const TpNodeT<T> &N = nodes0[n0 + j];
-                        ps_g[j][e] = tp_pse_node<T>(N, eh[ic0], lv[e] * N.ks, llv[e] + N.lnks);
-                    } else {
-                        const int ic = ics[e / kCacheEll];
-                        const TpNodeT<T> &N = nodes[(size_t)ic * TP_NNODES + n0 + j];
-                        ps_g[j][e] = tp_pse_node<T>(N, eh[ic], lv[e] * N.ks, llv[e] + N.lnks);
-                    }
+                    const int ic = set_ic[e < nu7 ? uset[e / 7] : 2 * ((e - nu7) / TP_NPTS_GM3)];
+                    const TpNodeT<T> &N = nodes[(size_t)ic * TP_NNODES + n0 + j];
+                    ps_g[j][e] = tp_pse_node<T>(N, eh[ic], lv[e] * N.ks, llv[e] + N.lnks);
                 }
             }
         }
@@ -480,15 +509,15 @@ static void launch_region_points(hipStream_t st, int lpp, const TpNodeT<T> *node
                            d_desc, d_fvals, mode, d_flag);
         break;
     case 16:
-        hipLaunchKernelGGL((k_region_cached<T, 1>), dim3((unsigned)((nreg + kCacheReg - 1) / kCacheReg)), dim3(256),
+        hipLaunchKernelGGL((k_region_cached<T, 1>), dim3((unsigned)((nreg + kCacheReg - 1) / kCacheReg)), dim3(kCacheThreads),
                            0, st, nodes, eh, nreg, d_reg, d_desc, d_fvals, mode, d_flag);
         break;
     case 32:
-        hipLaunchKernelGGL((k_region_cached<T, 2>), dim3((unsigned)((nreg + kCacheReg - 1) / kCacheReg)), dim3(512),
+        hipLaunchKernelGGL((k_region_cached<T, 2>), dim3((unsigned)((nreg + kCacheReg - 1) / kCacheReg)), dim3(2 * kCacheThreads),
                            0, st, nodes, eh, nreg, d_reg, d_desc, d_fvals, mode, d_flag);
         break;
     case 64:
-        hipLaunchKernelGGL((k_region_cached<T, 4>), dim3((unsigned)((nreg + kCacheReg - 1) / kCacheReg)), dim3(1024),
+        hipLaunchKernelGGL((k_region_cached<T, 4>), dim3((unsigned)((nreg + kCacheReg - 1) / kCacheReg)), dim3(4 * kCacheThreads),
                            0, st, nodes, eh, nreg, d_reg, d_desc, d_fvals, mode, d_flag);
         break;
     default:
@@ -557,7 +586,7 @@ static void region_points_shape(int lpp, size_t nreg, void **func, dim3 *grid, d
         *func = lpp == 16 ? (void *)k_region_cached<T, 1> : lpp == 32 ? (void *)k_region_cached<T, 2>
                                                                        : (void *)k_region_cached<T, 4>;
         *grid = dim3((unsigned)((nreg + kCacheReg - 1) / kCacheReg));
-        *block = dim3(16 * lpp);
+        *block = dim3(kCacheThreads * lpp / 16);
         break;
     default:
         *func = (void *)k_region_points<T, 1>;
