@@ -4,17 +4,19 @@
 // of them are most of its instructions.  Measured on one MI355X in units of one v_fma_f64 issue (2.03 ns per
 // wave and SIMD; 8 independent chains per thread, 8192 waves):
 //     exp 20, log 74, log1p 104, pow 161, x / y 13    (device library, compiler's IEEE division)
-//     tp_fp64_exp 14, tp_fp64_log 25, tp_fp64_rcp 6    (here)
+//     tp_fp64_exp 14, tp_fp64_log 18, tp_fp64_rcp 6    (here)
 // What is left out is what the node arithmetic never needs: a second word of the logarithm (every one feeds an
-// exponent or a sum whose own rounding is larger), the exactly rounded quotient, and branches for arguments
-// outside the range.  Domain: exp takes any finite argument below 2^31 in magnitude (it overflows to +inf and
-// underflows to 0 there like the library's), log any positive finite one (zeros, negative numbers and
-// infinities are stopped before the node loop; a NaN stays a NaN), rcp any normal number whose reciprocal is
-// normal.  Errors against 80-bit arithmetic: exp 0.91 ulp, log 0.93, log1p 1.17, exp10 1.19, rcp 0.50 (tests/test_fp64_math.py).
+// exponent or a sum whose own rounding is larger), the exactly rounded quotient, and branches for arguments outside the
+// range.  Domain: exp takes any finite argument below 2^31 in magnitude (it overflows to +inf and underflows to 0 there
+// like the library's; a NaN stays a NaN), log any positive normal one (a zero, a denormal, an infinity or a NaN gives
+// some finite number: where one can arrive, another factor of the same value carries it on), rcp any normal number whose
+// reciprocal is normal.  Errors against 80-bit arithmetic: exp 0.91 ulp, exp10 1.19, rcp 0.50, log 0.50 ulp + 2^-60
+// (tests/test_fp64_math.py).  The logarithm's table is there because its other form, 2 atanh((m - 1) / (m + 1)) with a
+// reciprocal and a degree-15 series, takes 31 instructions to these 15 (25 issues to 18).
 //
-// The coefficients are Chebyshev interpolants of (e^r - 1 - r) / r^2 on |r| <= ln 2 / 2 (degree 9) and of
-// 2 (atanh(s) / s - 1) / s^2 on |s| <= (sqrt 2 - 1) / (sqrt 2 + 1) (degree 6 in s^2), solved in 60-digit
-// arithmetic and rounded; relative remainders 1.6e-17 and 4.6e-18.
+// The coefficients of exp are the Chebyshev interpolant of (e^r - 1 - r) / r^2 on |r| <= ln 2 / 2 (degree 9), solved in
+// 60-digit arithmetic and rounded, relative remainder 1.6e-17; those of log that of (ln(1 + r) - r) / r^2 on
+// |r| < 0.00397 (degree 4), absolute remainder 1.4e-19.
 #pragma once
 #include <cmath>
 #include <cstring>
@@ -83,59 +85,58 @@ __host__ __device__ __forceinline__ double tp_fp64_rcp(double x)
     return fma(r, fma(e, e, e), r);
 }
 
-// k ln 2 + ln(1 + f) for 1 + f in [sqrt(1/2), sqrt(2)): with s = f / (2 + f), ln(1 + f) = 2 atanh(s) =
-// f - s (f - z P(z)), z = s^2; f is exact, and the rounding of s enters weighted by |f - z P| < 0.42
-__host__ __device__ __forceinline__ double tp_fp64_log_kf(double k, double f)
-{
-    const double s = f * tp_fp64_rcp(f + 2.0);
-    const double z = s * s;
-    double p = 0x1.2b5900de53b32p-3;
-    p = fma(p, z, 0x1.39fe51a7c18f9p-3);
-    p = fma(p, z, 0x1.7462b51cb66b1p-3);
-    p = fma(p, z, 0x1.c71c62e3f11e6p-3);
-    p = fma(p, z, 0x1.2492492df281ap-2);
-    p = fma(p, z, 0x1.99999999952d7p-2);
-    p = fma(p, z, 0x1.5555555555558p-1);
-    const double q = fma(-s, fma(-z, p, f), k * 0x1.abc9e3b39803fp-56);
-    return fma(k, 0x1.62e42fefa39efp-1, f + q);
-}
-
-__host__ __device__ __forceinline__ void tp_fp64_split(double x, double *m, int *k)
-{
-#ifdef TP_FP64_DEVICE
-    *m = __builtin_amdgcn_frexp_mant(x);
-    *k = __builtin_amdgcn_frexp_exp(x);
-#else
-    *m = std::frexp(x, k);
+// {c, -ln c} per interval of the mantissa (see the table's head); read per lane, 2 KB that stay in the vector L1
+#if defined(__HIP__) || defined(__HIPCC__)
+static __device__ const double tp_fp64_logtab[128][2] = {
+#include "tp_fp64_logtab.inc"
+};
 #endif
-    const bool lo = *m < 0x1.6a09e667f3bcdp-1;
-    *m = lo ? *m + *m : *m;
-    *k = lo ? *k - 1 : *k;
-}
+#ifndef TP_FP64_DEVICE
+static const double tp_fp64_logtab_host[128][2] = {
+#include "tp_fp64_logtab.inc"
+};
+#endif
 
+// ln x = k ln 2 - ln c + ln(1 + r), x = 2^k m, r = m c - 1, |r| < 0.004: with ln 2 and -ln c on multiples of 2^-43 the
+// first two add exactly; the rest is a degree-6 sum.  Absolute error half an ulp of the result + 2^-60 (near x = 1 that
+// is absolute, not relative: a caller that needs ln(1 + x) of a small x to its last bit does not use this).
 __host__ __device__ __forceinline__ double tp_fp64_log(double x)
 {
+#ifdef TP_FP64_DEVICE
+    const unsigned hi = (unsigned)__double2hiint(x);
+    const double k = __hiloint2double(0x43300000, (int)(hi >> 20)) - (0x1p52 + 1023.0);
+    const double m = __hiloint2double((int)((hi & 0xfffffu) | 0x3ff00000u), __double2loint(x));
+    const double *t = tp_fp64_logtab[(hi >> 13) & 127u];
+#else
+    unsigned long long b;
+    std::memcpy(&b, &x, 8);
+    const double k = (double)(b >> 52) - 1023.0;
+    const unsigned long long mb = (b & 0xfffffffffffffULL) | 0x3ff0000000000000ULL;
     double m;
-    int k;
-    tp_fp64_split(x, &m, &k);
-    return tp_fp64_log_kf((double)k, m - 1.0);
+    std::memcpy(&m, &mb, 8);
+    const double *t = tp_fp64_logtab_host[(b >> 45) & 127u];
+#endif
+    const double r = fma(m, t[0], -1.0);
+    double p = fma(r, -0x1.55569fde167adp-3, 0x1.999b135a6dab0p-3);
+    p = fma(p, r, -0x1.ffffffffaaa5ap-3);
+    p = fma(p, r, 0x1.55555555248f7p-2);
+    p = fma(p, r, -0.5);
+    const double q = fma(k, 0x1.ef35793c76730p-45, fma(r * r, p, r));
+    return fma(k, 0x1.62e42fefa3800p-1, t[1]) + q;
 }
 
-// ln(1 + x) for x >= 0 (or a NaN): ln u, u = 1 + x rounded, plus the rounding's share (x - (u - 1)) / u
+// ln(1 + x) for x >= 0 with the same absolute error: ln u, u = 1 + x rounded, plus the rounding's share
+// (x - (u - 1)) / u
 __host__ __device__ __forceinline__ double tp_fp64_log1p(double x)
 {
     const double u = 1.0 + x;
-    double m;
-    int k;
-    tp_fp64_split(u, &m, &k);
-    const double f = m - 1.0;
     const double c = u > 2.0 ? 1.0 - (u - x) : x - (u - 1.0);
 #ifdef TP_FP64_DEVICE
     const double r = __builtin_amdgcn_rcp(u);
 #else
     const double r = 1.0 / u;
 #endif
-    return tp_fp64_log_kf((double)k, f) + c * r;
+    return tp_fp64_log(u) + c * r;
 }
 
 // 10^x, |x| < 2^28: x = n log10 2 + r, the remainder taken in decades, so that the product by ln 10 rounds a small

@@ -346,7 +346,8 @@ __device__ __forceinline__ float tp_limber_pk_node32(const TpPNode32 &N, float e
 // are all of T1's work and are bound by FP64 issue, so a node takes the fewest instructions its factors allow: the
 // node's constants folded, the quotients merged, the damping in the exponent of (1 + Delta^2)^beta, and 1 / k^3 in
 // that of the T17 factor, whose logarithms need no more than their absolute rounding.  A T1 covariance of 210 pairs,
-// one MI355X: 155 ms with the library's functions, 81 with those of tp_fp64.h, 73-75 in this form.
+// one MI355X: 155 ms with the library's functions, 81 with those of tp_fp64.h, 73-75 in this form, 64 with the logarithm's
+// table.
 __host__ __device__ __forceinline__ double tp_limber_pk_node(const TpCosmoConst &C, const TpPNode &N, double ell,
                                                              double lell, int flags)
 {
