@@ -485,3 +485,24 @@ def test_non_finite_point_is_refused_and_leaves_no_flag(fid_tables, n):
         with pytest.raises(tp.TpError, match="non-finite"):
             call()
         assert np.array_equal(fid_tables.map3_integrand(x, th), good)
+
+
+@pytest.mark.parametrize("n_z, kw, tabulated", [
+    (3, {}, False), (41, dict(om=0.2, sigma8=0.7, ns=0.92, w=-1.2), False), (57, dict(om=0.45, sigma8=1.2, w=-0.7), False),
+    (33, dict(h=0.6), True)])
+def test_tables_of_other_grids_match_oracle(gpu_ctx, n_z, kw, tabulated):
+    """Growth (16 lanes a bin: 4 bins a wave, so odd grids leave a partial wave) and r_sigma (dyadic trapezoid levels,
+    short FP64 forms in the bisection) away from the fiducial grid, and with a tabulated P(k), at the table tolerance
+    1e-9; r_sigma, the end of the same bisection, to the last few bits."""
+    from _oracle import Oracle
+    c = tp.Cosmology(**dict(dict(zmax=3.0), **kw))
+    nz = W.resample_n_of_z(*W.nz_file_rows(), n_bins=n_z)
+    pk = None
+    if tabulated:
+        k = np.exp(np.linspace(np.log(1e-4), np.log(50.0), 400))
+        pk = (k, 2e4 * (k / 0.02) / (1 + (k / 0.02) ** 2.6))
+    t = tp.CosmologyTables([W.fiducial(), c, W.fiducial()], nz, n_z, 3.0, gpu_ctx, pk=pk)
+    g, o = t.tables(1), Oracle(c, nz, n_z, 3.0, pk=pk).tables()
+    for name in ["f_K", "g", "D1", "r_sigma", "n_eff", "ncur"]:
+        assert np.max(np.abs(g[name] - o[name]) / np.maximum(np.abs(o[name]), 1e-12)) < 1e-9, name
+    assert np.max(rel(g["r_sigma"], o["r_sigma"])) < 1e-14

@@ -7,16 +7,16 @@
 // (:676-707, bracket + bisection) and sigmam (:709-767, nested doubling
 // trapezoid in ln k).  The trapezoid sums inside sigmam are split over the 64
 // lanes of a wavefront and combined by an xor-butterfly, so every lane holds the
-// same sum and the bisection's control flow stays wave-uniform.
+// same sum and the bisection's control flow stays wave-uniform; a range's points up
+// to n = 64 are evaluated once, one per lane, for all its levels.
 //
 // Kernels (one stream, in order):
 //   k_cosmo_const   1 thread / cosmology   : derived constants, EH constants
 //   k_norm          1 wave / cosmology     : norm = sigma8 / sigma_TH(8)
 //   k_fK            1 thread / (cosmo,bin) : f_K(z_i)
 //   k_g             1 thread / (cosmo,bin) : g(z_i)
-//   k_lgr0          1 thread / cosmology   : lgr(0)
-//   k_d1            1 thread / (cosmo,bin) : D1 = lgr(z_i) / lgr(0)
-//   k_growth        1 wave / (cosmo,bin)   : r_sigma, n_eff, ncur
+//   k_lgr           16 lanes / (cosmo,bin) : lgr(z_i); bin 0 is z = 0
+//   k_growth        1 wave / (cosmo,bin)   : D1 = lgr(z_i) / lgr(0), r_sigma, n_eff, ncur
 //   k_nodes         1 thread / (cosmo,node): 96-node Limber tables (FP64 + FP32 copy)
 #include <algorithm>
 #include <cfloat>
@@ -24,7 +24,7 @@
 #include <string>
 #include <vector>
 
-#include "tp_device.h"
+#include "tp_power_dev.h"
 
 namespace {
 
@@ -39,11 +39,13 @@ __device__ __forceinline__ double window(double x, int i)
     return x * x * (1 - x * x) * exp(-x * x);
 }
 
-__device__ __forceinline__ double sigma_term(const TpCosmoConst &C, double k, double r, int j, double norm)
+// sigmam's integrand k^3 P(k) W(k r)^2 (W once for j = 3) as a product p w, the form in which its additions are fused
+__device__ __forceinline__ void sigma_pair(const TpCosmoConst &C, double k, double r, int j, double norm, double *p,
+                                           double *w)
 {
-    double w = window(k * r, j);
-    double kk = k * k * k * tp_pk_lin(C, k, norm);
-    return (j < 3) ? kk * w * w : kk * w;
+    *w = window(k * r, j);
+    const double kk = k * k * k * tp_pk_lin(C, k, norm);
+    *p = (j < 3) ? kk * *w : kk;
 }
 
 __device__ __forceinline__ double wave_sum(double v)
@@ -53,25 +55,71 @@ __device__ __forceinline__ double wave_sum(double v)
     return v;
 }
 
-// sigmam with lane-split trapezoid sums; all 64 lanes call it with equal arguments.
+// The points of the dyadic levels n = 2, 4, ..., 64 of a trapezoid, one per lane: lane l >= 1 holds the odd index o of
+// the level m = 2 2^floor(log2 l), so the levels' odd points lie in lanes [m / 2, m).  Level n's point i = o 2^t is level
+// n / 2^t's odd point o with the same bits, its step being an exact power of two times the finer one.
+__device__ __forceinline__ void dyadic_point(int lane, int *m, int *o)
+{
+    const int half = lane ? 1 << (31 - __clz(lane)) : 1;
+    *m = 2 * half;
+    *o = lane ? 2 * (lane - half) + 1 : 1;
+}
+
+// sigmam with lane-split trapezoid sums; all 64 lanes call it with equal arguments.  The reference evaluates every point
+// of every level anew; here a range's levels up to 64 share one evaluation per lane, the ends of the first eight ranges
+// another, and the sums keep the order of the plain form (lane i - 1 holds point i, then the butterfly), bit for bit.
 __device__ double sigmam_wave(const TpCosmoConst &C, double r, int j, double norm, int lane)
 {
     const double eps = 1.e-4;
     double k1 = 2. * kPi / r, k2 = 2. * kPi / r;
+    double ep, ew;  // lane 2 q: lower end of range q < 8, lane 2 q + 1: upper end
+    {
+        double e1 = k1, e2 = k2;
+        for (int q = 0; q < 8; ++q)
+            if (q <= lane >> 1) {
+                e1 = e1 / 10.0;
+                e2 = e2 * 2.0;
+            }
+        sigma_pair(C, lane & 1 ? e2 : e1, r, j, norm, &ep, &ew);
+    }
+    int m, o;
+    dyadic_point(lane, &m, &o);
     double xx = 0, xxpp = -1.0;
     for (int outer = 0; outer < 30; ++outer) {  // bounded; converges after a few range doublings
         k1 = k1 / 10.0;
         k2 = k2 * 2.0;
         double a = log(k1), b = log(k2);
+        double p, w, p1, w1, p2, w2;
+        sigma_pair(C, exp(a + (b - a) / (double)m * o), r, j, norm, &p, &w);
+        const double term = lane ? p * w : 0.0;
+        if (outer < 8) {
+            p1 = __shfl(ep, 2 * outer, 64);
+            w1 = __shfl(ew, 2 * outer, 64);
+            p2 = __shfl(ep, 2 * outer + 1, 64);
+            w2 = __shfl(ew, 2 * outer + 1, 64);
+        } else {
+            sigma_pair(C, k1, r, j, norm, &p1, &w1);
+            sigma_pair(C, k2, r, j, norm, &p2, &w2);
+        }
+        const double ends = 0.5 * (p1 * w1 + p2 * w2);
         double xxp = -1.0;
         int n = 2;
         for (int inner = 0; inner < 22; ++inner) {  // n <= 2^23
             n = n * 2;
             double hh = (b - a) / (double)n;
             double part = 0.;
-            for (int i = 1 + lane; i < n; i += 64) part += sigma_term(C, exp(a + hh * i), r, j, norm);
+            if (n <= 64) {
+                const int i = lane + 1, t = __ffs(i) - 1;  // i = o 2^t
+                const int src = i < n ? (n >> t >> 1) + (((i >> t) - 1) >> 1) : 0;
+                part = __shfl(term, src, 64);
+            } else {
+                for (int i = 1 + lane; i < n; i += 64) {
+                    sigma_pair(C, exp(a + hh * i), r, j, norm, &p, &w);
+                    part += p * w;
+                }
+            }
             xx = wave_sum(part);
-            xx += 0.5 * (sigma_term(C, k1, r, j, norm) + sigma_term(C, k2, r, j, norm));
+            xx += ends;
             xx *= hh;
             if (fabs((xx - xxp) / xx) < eps) break;
             xxp = xx;
@@ -83,18 +131,84 @@ __device__ double sigmam_wave(const TpCosmoConst &C, double r, int j, double nor
     return xx / (2.0 * kPi * kPi);
 }
 
-__device__ double lgr_func1(const TpCosmoConst &C, double la, const double y[2])
+// sigmam for the bisection of r_sigma (j = 1), where only comparisons with 1 and the levels' convergence are read: the
+// same points, ranges and tests with the short FP64 forms and the levels' sums taken as sums of their odd points.  Its
+// value (C.norm included) differs from sigmam_wave's by rounding; a decision would differ only for a quantity within ~1e-14 of its bound.
+__device__ __forceinline__ double sigma_delta(const TpCosmoConst &C, double lk, double r)
+{
+    const double k = tp_fp64_exp(lk), x = k * r;
+    const double d = tp_delta2_lin(C, 1.0, k, lk);
+    return d * tp_fp64_exp(fmax(-x * x, -1000.0));  // W^2 = exp(-x^2)
+}
+__device__ double sigma_bisect(const TpCosmoConst &C, double r, int lane)
+{
+    const double eps = 1.e-4;
+    double k1 = 2. * kPi / r, k2 = k1;
+    double e1 = k1, e2 = k1;
+    for (int q = 0; q < 8; ++q)
+        if (q <= lane >> 1) {
+            e1 = e1 * 0.1;
+            e2 = e2 * 2.0;
+        }
+    const double ev = sigma_delta(C, tp_fp64_log(lane & 1 ? e2 : e1), r);
+    int m, o;
+    dyadic_point(lane, &m, &o);
+    const double fo = (double)o / (double)m;  // exact
+    double xx = 0, xxpp = -1.0;
+    for (int outer = 0; outer < 30; ++outer) {
+        k1 = k1 * 0.1;
+        k2 = k2 * 2.0;
+        const double a = tp_fp64_log(k1), b = tp_fp64_log(k2);
+        double v = lane ? sigma_delta(C, fma(b - a, fo, a), r) : 0.0;
+        for (int s = 16; s >= 1; s >>= 1) {  // sums within each level's lanes [m / 2, m)
+            const double u = __shfl_xor(v, s, 64);
+            if (lane >= 2 * s) v += u;
+        }
+        const double ends = outer < 8 ? __shfl(ev, 2 * outer, 64) + __shfl(ev, 2 * outer + 1, 64)
+                                      : sigma_delta(C, a, r) + sigma_delta(C, b, r);
+        double T = __shfl(v, 1, 64) + 0.5 * ends;
+        double xxp = -1.0;
+        int n = 2;
+        for (int inner = 0; inner < 22; ++inner) {
+            n = n * 2;
+            const double hh = (b - a) / (double)n;
+            if (n <= 64) {
+                T += __shfl(v, n >> 1, 64);
+            } else {
+                double part = 0.;
+                for (int i = 1 + 2 * lane; i < n; i += 128) part += sigma_delta(C, fma(hh, (double)i, a), r);
+                T += wave_sum(part);
+            }
+            xx = T * hh;
+            if (fabs((xx - xxp) / xx) < eps || isnan(xx)) break;
+            xxp = xx;
+        }
+        if (fabs((xx - xxpp) / xx) < eps || isnan(xx)) break;
+        xxpp = xx;
+    }
+    return sqrt(xx);
+}
+
+// a^(-3 w) at ln a, the ODE's only transcendental
+__device__ __forceinline__ double lgr_aw(const TpCosmoConst &C, double la)
+{
+    double a = exp(la);
+    return pow(a, -3. * C.w);
+}
+
+__device__ __forceinline__ double lgr_func1(const TpCosmoConst &C, double aw, const double y[2])
 {
     // classed_version/bispectrum.cpp:895-907 (j == 1)
-    double a = exp(la);
-    double aw = pow(a, -3. * C.w);
     double g = -0.5 * (5. * C.om + (5. - 3 * C.w) * C.ow * aw) * y[1] - 1.5 * (1. - C.w) * C.ow * aw * y[0];
     return g / (C.om + C.ow * aw);
 }
 
-__device__ double lgr(const TpCosmoConst &C, double z)
+// lgr(z), classed_version/bispectrum.cpp:843-893: RK4 in ln a, n = 20, 40, ... steps until rel 1e-5.  The steps are one
+// serial chain, but a^(-3w) at their ends and midpoints is not part of it: kLgrLanes lanes that call this with the same
+// z take one such point each and pass it round by shuffles, eight steps at a time.
+constexpr int kLgrLanes = 16;
+__device__ double lgr(const TpCosmoConst &C, double z, int lane16)
 {
-    // classed_version/bispectrum.cpp:843-893: RK4 in ln a, n = 20, 40, ... until rel 1e-5
     double a = 1. / (1. + z), a0 = 1. / 1100.;
     double yp = -1., y0 = 0;
     int n = 10;
@@ -102,26 +216,35 @@ __device__ double lgr(const TpCosmoConst &C, double z)
         n *= 2;
         double h = (log(a) - log(a0)) / n;
         double x = log(a0);
+        double aw0 = lgr_aw(C, x);
         double y[2] = {1., 0.};
-        for (int i = 0; i < n; i++) {
-            double k1[2], k2[2], k3[2], k4[2], yt[2];
-            k1[0] = h * y[1];
-            k1[1] = h * lgr_func1(C, x, y);
-            yt[0] = y[0] + 0.5 * k1[0];
-            yt[1] = y[1] + 0.5 * k1[1];
-            k2[0] = h * yt[1];
-            k2[1] = h * lgr_func1(C, x + 0.5 * h, yt);
-            yt[0] = y[0] + 0.5 * k2[0];
-            yt[1] = y[1] + 0.5 * k2[1];
-            k3[0] = h * yt[1];
-            k3[1] = h * lgr_func1(C, x + 0.5 * h, yt);
-            yt[0] = y[0] + k3[0];
-            yt[1] = y[1] + k3[1];
-            k4[0] = h * yt[1];
-            k4[1] = h * lgr_func1(C, x + h, yt);
-            y[0] += (k1[0] + k4[0]) / 6. + (k2[0] + k3[0]) / 3.;
-            y[1] += (k1[1] + k4[1]) / 6. + (k2[1] + k3[1]) / 3.;
-            x += h;
+        for (int i0 = 0; i0 < n; i0 += kLgrLanes / 2) {
+            double xs = x;  // the start of step i0 + lane16 / 2, by the chain's own additions
+            for (int t = 0; t < kLgrLanes / 2 - 1; ++t)
+                if (t < lane16 >> 1) xs += h;
+            const double awl = lgr_aw(C, lane16 & 1 ? xs + 0.5 * h : xs + h);
+            for (int s = 0; s < kLgrLanes / 2 && i0 + s < n; ++s) {
+                const double awm = __shfl(awl, 2 * s + 1, kLgrLanes), aw1 = __shfl(awl, 2 * s, kLgrLanes);
+                double k1[2], k2[2], k3[2], k4[2], yt[2];
+                k1[0] = h * y[1];
+                k1[1] = h * lgr_func1(C, aw0, y);
+                yt[0] = y[0] + 0.5 * k1[0];
+                yt[1] = y[1] + 0.5 * k1[1];
+                k2[0] = h * yt[1];
+                k2[1] = h * lgr_func1(C, awm, yt);
+                yt[0] = y[0] + 0.5 * k2[0];
+                yt[1] = y[1] + 0.5 * k2[1];
+                k3[0] = h * yt[1];
+                k3[1] = h * lgr_func1(C, awm, yt);
+                yt[0] = y[0] + k3[0];
+                yt[1] = y[1] + k3[1];
+                k4[0] = h * yt[1];
+                k4[1] = h * lgr_func1(C, aw1, yt);
+                y[0] += (k1[0] + k4[0]) / 6. + (k2[0] + k3[0]) / 3.;
+                y[1] += (k1[1] + k4[1]) / 6. + (k2[1] + k3[1]) / 3.;
+                x += h;
+                aw0 = aw1;
+            }
         }
         y0 = y[0];
         if (fabs(y0 / yp - 1.) < 0.1 * 1.e-4) break;
@@ -366,45 +489,50 @@ __global__ void k_g(int ncosmo, int n_z, double dz, double z_max, const double *
     tab[(size_t)ic * 6 * n_z + n_z + i] = g;
 }
 
-// lgr(0) of each cosmology, one thread per cosmology (every z-bin's D1 divides by it)
-__global__ void k_lgr0(int ncosmo, const TpCosmoConst *cc, double *lgr0)
+// lgr(z_i) of each (cosmology, z-bin); bin 0 (z = 0) is what every D1 divides by
+__global__ void __launch_bounds__(64) k_lgr(int ncosmo, int n_z, double dz, const TpCosmoConst *cc, double *raw)
 {
-    const int ic = blockIdx.x * blockDim.x + threadIdx.x;
-    if (ic < ncosmo) lgr0[ic] = lgr(cc[ic], 0.);
+    const int t = (blockIdx.x * 64 + threadIdx.x) / kLgrLanes, l = threadIdx.x % kLgrLanes;
+    if (t >= ncosmo * n_z) return;  // whole groups of kLgrLanes lanes
+    double z;
+    {
+#pragma clang fp contract(off)  // z_i = i dz is a rounded number of its own, not part of 1 + z
+        z = t % n_z * dz;
+    }
+    const double v = lgr(cc[t / n_z], z, l);
+    if (l == 0) raw[t] = v;
 }
 
-// D1 = lgr(z) / lgr(0) (classed_version/bispectrum.cpp:157), one thread per (cosmology, z-bin): the growth
-// ODE is sequential, so each lane integrates its own bin instead of a whole wave repeating one
-__global__ void k_d1(int ncosmo, int n_z, double dz, const TpCosmoConst *cc, const double *lgr0, double *tab)
-{
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= ncosmo * n_z) return;
-    const int ic = t / n_z, i = t % n_z;
-    tab[(size_t)ic * 6 * n_z + 2 * n_z + i] = lgr(cc[ic], i * dz) / lgr0[ic];
-}
-
-// r_sigma, n_eff and ncur of one (cosmology, z-bin) per wave, from the bin's D1
-__global__ void __launch_bounds__(64) k_growth(int ncosmo, int n_z, double dz, const TpCosmoConst *cc, double *tab)
+// D1, r_sigma, n_eff and ncur of one (cosmology, z-bin) per wave.  ~25 sigma(R) of ~4 ranges each: every level of every
+// range evaluated anew, with its ends, by the library's pow and log was ~60 wave passes of ~700 instructions per sigma(R)
+// (46 ms for 512 cosmologies, 1.6 ms for one); one pass per range, and ~150 instructions a pass in the bisection, is 9 ms
+// and 0.25 ms.  Same bits in every table.
+__global__ void __launch_bounds__(64) k_growth(int ncosmo, int n_z, double dz, const TpCosmoConst *cc,
+                                               const double *raw, double *tab)
 {
     int ic = blockIdx.x / n_z, i = blockIdx.x % n_z;
     if (ic >= ncosmo) return;
     int lane = threadIdx.x;
-    TpCosmoConst C = cc[ic];
+    const TpCosmoConst &C = cc[ic];
     const double eps = 1.e-4;
-    const double D1 = tab[(size_t)ic * 6 * n_z + 2 * n_z + i];
-    // calc_r_sigma, classed_version/bispectrum.cpp:676-707
+    const double D1 = raw[(size_t)ic * n_z + i] / raw[(size_t)ic * n_z];  // classed_version/bispectrum.cpp:157
+    // calc_r_sigma, classed_version/bispectrum.cpp:676-707 (far outside any r_sigma the short forms could leave their
+    // range: there a bracket that does not close ends as the plain form ends it)
+    auto sigma1 = [&](double q) {
+        return q > 1e-8 && q < 1e8 ? sigma_bisect(C, 1. / q, lane) : sigmam_wave(C, 1. / q, 1, C.norm, lane);
+    };
     double k, k1 = 1., k2 = 1.;
     for (int it = 0; it < 200; ++it) {
-        if (D1 * sigmam_wave(C, 1. / k1, 1, C.norm, lane) < 1.) break;
+        if (D1 * sigma1(k1) < 1.) break;
         k1 *= 0.5;
     }
     for (int it = 0; it < 200; ++it) {
-        if (D1 * sigmam_wave(C, 1. / k2, 1, C.norm, lane) > 1.) break;
+        if (D1 * sigma1(k2) > 1.) break;
         k2 *= 2.;
     }
     for (int it = 0; it < 400; ++it) {
         k = 0.5 * (k1 + k2);
-        double s = D1 * sigmam_wave(C, 1. / k, 1, C.norm, lane);
+        double s = D1 * sigma1(k);
         if (s < 1.)
             k1 = k;
         else if (s > 1.)
@@ -417,6 +545,7 @@ __global__ void __launch_bounds__(64) k_growth(int ncosmo, int n_z, double dz, c
     double d1 = -2. * (D1 * s2) * (D1 * s2);
     if (lane == 0) {
         double *T = tab + (size_t)ic * 6 * n_z;
+        T[2 * n_z + i] = D1;
         T[3 * n_z + i] = rs;
         T[4 * n_z + i] = -3. + 2. * (D1 * s2) * (D1 * s2);   // classed_version/bispectrum.cpp:160
         T[5 * n_z + i] = d1 * d1 + 4. * s3 * D1 * D1;          // :161
@@ -667,7 +796,7 @@ static int cosmo_build(tp_ctx *ctx, int ncosmo, const tp_cosmology *params, cons
     const size_t o_eh32 = take(sizeof(TpEH32) * (size_t)ncosmo);
     const size_t o_base32 = take(sizeof(TpNode32) * TP_NBASE * (size_t)ncosmo);
     const size_t o_err = take(sizeof(int));
-    const size_t o_params = take(sizeof(tp_cosmology) * ncosmo + sizeof(double) * ncosmo);
+    const size_t o_params = take(sizeof(tp_cosmology) * ncosmo + sizeof(double) * n_z * (size_t)ncosmo);
     const size_t o_pk = nk ? take((2 * nkt + 2 * (size_t)ncosmo) * sizeof(double) + ngt * sizeof(int)) : 0;
     TPC(hipMalloc(&c->d_arena, off));
     char *arena = (char *)c->d_arena;
@@ -698,7 +827,7 @@ static int cosmo_build(tp_ctx *ctx, int ncosmo, const tp_cosmology *params, cons
         TPC(hipMemcpy(d_idx, hidx.data(), ngt * sizeof(int), hipMemcpyHostToDevice));
     }
     tp_cosmology *d_params = (tp_cosmology *)(arena + o_params);
-    double *d_lgr0 = (double *)(d_params + ncosmo);  // lgr(0) per cosmology
+    double *d_lgr = (double *)(d_params + ncosmo);  // lgr(z_i) per cosmology and bin
     TPC(hipMemcpyAsync(d_params, params, sizeof(tp_cosmology) * ncosmo, hipMemcpyHostToDevice, s));
     // n(z) of every cosmology in one copy (the stream is synchronised before h_nz goes out of scope)
     std::vector<double> h_nz((size_t)ncosmo * n_z);
@@ -716,9 +845,9 @@ static int cosmo_build(tp_ctx *ctx, int ncosmo, const tp_cosmology *params, cons
     hipLaunchKernelGGL(k_fK, dim3((nt + 127) / 128), dim3(128), 0, s, ncosmo, n_z, dz, c->d_const, c->d_tab,
                        c->d_err);
     hipLaunchKernelGGL(k_g, dim3((nt + 127) / 128), dim3(128), 0, s, ncosmo, n_z, dz, z_max, c->d_nz, c->d_tab);
-    hipLaunchKernelGGL(k_lgr0, dim3((ncosmo + 63) / 64), dim3(64), 0, s, ncosmo, c->d_const, d_lgr0);
-    hipLaunchKernelGGL(k_d1, dim3((nt + 63) / 64), dim3(64), 0, s, ncosmo, n_z, dz, c->d_const, d_lgr0, c->d_tab);
-    hipLaunchKernelGGL(k_growth, dim3(nt), dim3(64), 0, s, ncosmo, n_z, dz, c->d_const, c->d_tab);
+    hipLaunchKernelGGL(k_lgr, dim3((unsigned)(((size_t)nt * kLgrLanes + 63) / 64)), dim3(64), 0, s, ncosmo, n_z, dz,
+                       c->d_const, d_lgr);
+    hipLaunchKernelGGL(k_growth, dim3(nt), dim3(64), 0, s, ncosmo, n_z, dz, c->d_const, d_lgr, c->d_tab);
     int nn = ncosmo * (TP_NNODES + TP_NBASE);
     hipLaunchKernelGGL(k_nodes, dim3((nn + 127) / 128), dim3(128), 0, s, ncosmo, n_z, c->d_const, c->d_tab,
                        c->d_node64, c->d_node32, c->d_eh64, c->d_eh32, c->d_base32);
