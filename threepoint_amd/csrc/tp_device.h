@@ -23,6 +23,13 @@ template <> struct TpMath<float> {
     static __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 };
 
+__device__ __forceinline__ float tp_logf_normal(float x)
+{
+    const float y = __builtin_amdgcn_logf(x), p = 0x1.62e42ep-1f * y;
+    const float e = __builtin_fmaf(0x1.efa39ep-25f, y, __builtin_fmaf(0x1.62e42ep-1f, y, -p));
+    return __builtin_fmaf(0x1.62e42ep-1f, y, e);
+}
+
 // The functions of the z-node arithmetic (the loops over nodes and Ogata terms), separate from those of the
 // per-point set-up: in FP64 the short forms of tp_fp64.h, in FP32 the native ones.  FP64 against the device
 // library's functions, one MI355X: 17 920 <Map^3> integrals 6.98 -> 4.71 s with the series logarithm, 10^6 B_kappa points 6.3 -> 4.8 ms,
@@ -32,12 +39,7 @@ template <class T> struct TpNodeMath : TpMath<T> {};
 template <> struct TpNodeMath<float> : TpMath<float> {
     // __logf without its branches for denormals and infinities (12 instructions to 5, same bits for x >= FLT_MIN):
     // ln 2 times v_log_f32, the product's rounding and the constant's second word added back
-    static __device__ __forceinline__ float lg(float x)
-    {
-        const float y = __builtin_amdgcn_logf(x), p = 0x1.62e42ep-1f * y;
-        const float e = __builtin_fmaf(0x1.efa39ep-25f, y, __builtin_fmaf(0x1.62e42ep-1f, y, -p));
-        return __builtin_fmaf(0x1.62e42ep-1f, y, e);
-    }
+    static __device__ __forceinline__ float lg(float x) { return tp_logf_normal(x); }
 };
 template <> struct TpNodeMath<double> {
     static __host__ __device__ __forceinline__ double ex(double x) { return tp_fp64_exp(x); }
@@ -115,7 +117,12 @@ __host__ __device__ __forceinline__ T tp_plin_q(const TpNodeT<T> &N, const TpEHT
     T d = T(1) + x2 * x2;
     T qeff = kk * E.theta2 * d * M::rcp(E.omh2 * (E.sqrt_alnu * d + E.one_m_sqrt_alnu));
     T L = M::lg(E.e_const + E.cL * qeff);
-    T den = T(1) + T(60.5) * M::ex(T(1.11) * M::lg(qeff));
+    T lqeff;
+    if constexpr (std::is_same<T, float>::value)  // below FLT_MIN the power is lost in the 1 either way
+        lqeff = M::lg(fmaxf(qeff, 0x1p-126f));
+    else
+        lqeff = M::lg(qeff);
+    T den = T(1) + T(60.5) * M::ex(T(1.11) * lqeff);
     T Ld = L * den;
     T r = Ld * M::rcp(Ld + (T(14.4) * den + T(325.0)) * qeff * qeff);
     return N.pk_pref * M::ex(E.three_ns * (lq + N.lnkoff) - T(3) * lq) * r * r;

@@ -252,19 +252,21 @@ __global__ void k_power_points(const TpCosmoConst *__restrict__ cc, const double
 // apertureStatisticsCovariance.cu:1958-1985) over whole 3-D regions (l1, l2, phi): the rule points are
 // generated and the Genz-Malik rule applied on the device, so a round moves one region record in and
 // one result out per region.  Of a region's 33 points only 7 distinct l1 (the axis-0 codes -3..3) and
-// 7 distinct l2 occur, so a region needs 7 + 7 + 33 = 47 Pell, not 99.  A workgroup takes kT1Reg
+// 7 distinct l2 occur, so a region needs 7 + 7 + 33 = 47 Pell, not 99.  A workgroup takes 4 or 5
 // regions in three phases:
 //   1. one thread per Pell (7 l1, 7 l2, 33 l3 per region; those of cut points skipped), the node order
 //      of pell_nodes, so each value has the bits of a per-point evaluation;
 //   2. one thread per point: the integrand from the cached Pell, in the reference's product order;
 //   3. one thread per region: the rule (gm_rule3, the host rule's arithmetic order).
-constexpr int kT1Reg = 4;                     // regions per workgroup: 188 Pell on 192 threads (98% of the lanes;
-                                              // 5 regions fill 235 of 256, 92%)
-constexpr int kT1Block = 192;
+// Regions per workgroup and its threads: FP64 4 on 192 (188 Pell, 98% of the lanes; 5 on 256 fill 92%); the FP32 form,
+// whose workgroups are short, keeps the larger ones (210 pairs: 28.9 ms, and 29.1 with 4 on 192; 26.3 since its nodes take the branch-free logarithm)
+template <bool F32> struct T1Shape {
+    static constexpr int reg = F32 ? 5 : 4, block = F32 ? 256 : 192;
+};
 constexpr int kT1Pell = 14 + TP_NPTS_GM3;     // Pell per region
 
 template <bool F32>  // F32: the Pell from the FP32 node records (pell_nodes32)
-__global__ void __launch_bounds__(kT1Block) k_t1_regions(const TpCosmoConst *__restrict__ cc,
+__global__ void __launch_bounds__(T1Shape<F32>::block) k_t1_regions(const TpCosmoConst *__restrict__ cc,
                                                     const TpPNode *__restrict__ pnode,
                                                     const TpPNode32 *__restrict__ pnode32, double dx,
                                                     const TpPowerDesc *__restrict__ desc,
@@ -272,6 +274,7 @@ __global__ void __launch_bounds__(kT1Block) k_t1_regions(const TpCosmoConst *__r
                                                     TpRegionOut *__restrict__ out)
 {
 #pragma clang fp contract(off)
+    constexpr int kT1Reg = T1Shape<F32>::reg;
     __shared__ double pl[kT1Reg][kT1Pell];
     __shared__ double fv[kT1Reg][TP_NPTS_GM3];
     const size_t r0 = (size_t)blockIdx.x * kT1Reg;
@@ -886,10 +889,12 @@ int t1_regions(tp_ctx *ctx, const tp_cosmo *c, const std::vector<TpPowerDesc> &d
 {
     auto launch = [&](size_t nreg, const TpRegion *d_reg, TpRegionOut *d_out, double *, hipStream_t st,
                       hipEvent_t evm) -> int {
-        const size_t nblk = (nreg + kT1Reg - 1) / kT1Reg;
+        const bool f32 = mode == TP_MODE_FP32;
+        const int nr = f32 ? T1Shape<true>::reg : T1Shape<false>::reg;
+        const size_t nblk = (nreg + nr - 1) / nr;
         if (nblk > 0x7fffffffu) return tp_set_error(TP_ECAPACITY, "T1: too many regions for one launch");
-        hipLaunchKernelGGL(mode == TP_MODE_FP32 ? k_t1_regions<true> : k_t1_regions<false>, dim3((unsigned)nblk),
-                           dim3(kT1Block), 0, st, c->d_const, (const TpPNode *)c->d_pnode,
+        hipLaunchKernelGGL(f32 ? k_t1_regions<true> : k_t1_regions<false>, dim3((unsigned)nblk),
+                           dim3(f32 ? T1Shape<true>::block : T1Shape<false>::block), 0, st, c->d_const, (const TpPNode *)c->d_pnode,
                            (const TpPNode32 *)c->d_pnode32, c->z_max / 2, (const TpPowerDesc *)ctx->d_desc.p, d_reg,
                            nreg, d_out);
         TP_HIP(hipGetLastError());

@@ -320,8 +320,8 @@ __device__ __forceinline__ float tp_limber_pk_node32(const TpPNode32 &N, float e
     const float kh = k * N.h, x = N.sh043 * kh, x2 = x * x;
     const float geff = N.omh2 * (N.sqa + (1.f - N.sqa) * __builtin_amdgcn_rcpf(1.f + x2 * x2));
     const float qeff = kh * __builtin_amdgcn_rcpf(geff) * N.theta2;
-    const float L = __logf(2.718281828f + N.cL * qeff);
-    const float Cq = 14.4f + 325.f * __builtin_amdgcn_rcpf(1.f + 60.5f * __expf(1.11f * __logf(qeff)));
+    const float L = tp_logf_normal(2.718281828f + N.cL * qeff);
+    const float Cq = 14.4f + 325.f * __builtin_amdgcn_rcpf(1.f + 60.5f * __expf(1.11f * tp_logf_normal(fmaxf(qeff, 0x1p-126f))));
     const float r = L * __builtin_amdgcn_rcpf(L + Cq * qeff * qeff);
     const float plin = r * r * __expf(N.ns3 * lk + N.ld);  // Delta^2_lin
     float P = plin;
@@ -330,14 +330,14 @@ __device__ __forceinline__ float tp_limber_pk_node32(const TpPNode32 &N, float e
         float ph = N.a * __expf(N.f1x3 * ly) *
                    __builtin_amdgcn_rcpf(1.f + N.b * __expf(N.f2 * ly) + __expf(N.gam3 * (N.lf3c + ly)));
         ph = ph * __builtin_amdgcn_rcpf(1.f + N.xnu * __builtin_amdgcn_rcpf(ysqr));
-        const float pq = plin * __expf(N.beta * __logf(1.f + plin)) * __builtin_amdgcn_rcpf(1.f + plin * N.alpha) *
+        const float pq = plin * __expf(N.beta * tp_logf_normal(1.f + plin)) * __builtin_amdgcn_rcpf(1.f + plin * N.alpha) *
                          __expf(-0.25f * y - 0.125f * ysqr);
         P = pq + ph;
     }
     float v = P * __expf(N.lp - 3.f * lk);
     if (flags & TP_PK_T17) {  // tp_t17_factor
         const float c1 = 9.5171e-4f, c2 = 5.1543e-3f, a1 = 1.3063f, a2 = 1.1475f, a3 = 0.62793f;
-        v *= __expf(a1 * __logf(1.f + c1 * __expf(-a1 * lk)) - a3 * __logf(1.f + c2 * __expf(-a2 * lk)));
+        v *= __expf(a1 * tp_logf_normal(1.f + c1 * __expf(-a1 * lk)) - a3 * tp_logf_normal(1.f + c2 * __expf(-a2 * lk)));
     }
     return v;
 }
