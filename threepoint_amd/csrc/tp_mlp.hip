@@ -77,113 +77,221 @@ static_assert(NPARAM == 199937, "parameter count");
 constexpr size_t OFF_W[3] = {OFF_W2, OFF_W3, OFF_W4};
 constexpr size_t OFF_B[3] = {OFF_B2, OFF_B3, OFF_B4};
 
-// --------------------------------------------------------------- MFMA GEMM
-// C[M][N] (+)= sum_k A(m,k) B(k,n), A and B BF16 addressed through strides, FP32 accumulation.
-// Block 256 threads = 4 waves; block tile 64x64; wave tile 32x32 (one 32x32x8 MFMA accumulator);
-// K staged through LDS in steps of 32 ([m][k] and [n][k] order, k contiguous for the MFMA).
-// Requires M % 64 == 0, N % 64 == 0, K % 32 == 0 (checked on the host).
-constexpr int BM = 64, BN = 64, BK = 32, KPAD = 8;
+// --------------------------------------------------------------- training GEMMs
+// The hidden layers of a training batch, BF16 operands with FP32 accumulation by 32x32x8 MFMAs, K ascending.  A batch of
+// 8192 rows is 1 GFLOP per product, a microsecond of matrix-core time: what counts is that operands arrive in 16-byte
+// loads, that the next stage's are in flight during the MFMAs, and how many launches a step takes (8192 rows forward and
+// backward: 577 us on the device with 2-byte loads, one launch per gradient and an atomic per row for the loss; @MLP@
+// in this form, gradients unchanged to the bit).
+constexpr int GM = 64, GN = 128, GK = 64, GPAD = 8;
 
-struct GemmArgs {
-    const unsigned short *A;
-    long long sam, sak;
-    const unsigned short *B;
-    long long sbk, sbn;
-    int M, N, K;
-    int kchunk;       // K range per blockIdx.z (split-K)
-    int epi;          // 0: FP32 partial C[z][M][N]; 1: forward bias+SiLU (+Z); 2: backward SiLU'; 3: inference
-    float *C;         // epi 0: partial outputs
-    const float *bias;
-    float *Z;         // epi 1: pre-activation out (FP32, [M][N]); epi 2: pre-activation in
-    unsigned short *Aout;  // epi 1: BF16 activation; epi 2: BF16 gradient w.r.t. pre-activation
-    int ldo;
-};
+__device__ __forceinline__ bf16x4 lds_frag(const unsigned short *p) { return *(const bf16x4 *)p; }
 
-__global__ void __launch_bounds__(256) k_gemm_bf16(GemmArgs g)
+// C[M][H] = sum_k A(m, k) B(n, k), both k-contiguous with row length H.  Tile 64 x 128, four waves of 32 x 64.
+// BWD false: Z = C + bias, out = bf16(SiLU(Z)).  BWD true: out = bf16(C SiLU'(Z)).  M % 64 == 0 (checked on the host).
+template <bool BWD>
+__global__ void __launch_bounds__(256) k_gemm_rows(const unsigned short *__restrict__ A,
+                                                   const unsigned short *__restrict__ B,
+                                                   const float *__restrict__ bias, float *__restrict__ Z,
+                                                   unsigned short *__restrict__ out)
 {
-    __shared__ unsigned short sA[BM][BK + KPAD];
-    __shared__ unsigned short sB[BN][BK + KPAD];
+    __shared__ __align__(16) unsigned short sA[GM][GK + GPAD], sB[GN][GK + GPAD];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int m0 = blockIdx.x * BM, n0 = blockIdx.y * BN;
-    const int kbeg = blockIdx.z * g.kchunk, kend = min(g.K, kbeg + g.kchunk);
-    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-    f32x16 acc;
-    for (int i = 0; i < 16; ++i) acc[i] = 0.f;
-    const bool a_kfast = (g.sak == 1), b_kfast = (g.sbk == 1);
-    for (int k0 = kbeg; k0 < kend; k0 += BK) {
-        // global -> LDS, consecutive threads on the contiguous dimension
+    const size_t m0 = (size_t)blockIdx.x * GM;
+    const int n0 = blockIdx.y * GN, wm = (wave >> 1) * 32, wn = (wave & 1) * 64;
+    const int lr = tid >> 3, lc = (tid & 7) * 8;  // this thread's row (of 32 per load) and first k
+    uint4 ra[2], rb[4];
+    auto fetch = [&](int k0) {
 #pragma unroll
-        for (int j = 0; j < (BM * BK) / 256; ++j) {
-            int e = tid + 256 * j;
-            int mm, kk;
-            if (a_kfast) { mm = e / BK; kk = e % BK; } else { kk = e / BM; mm = e % BM; }
-            sA[mm][kk] = g.A[(long long)(m0 + mm) * g.sam + (long long)(k0 + kk) * g.sak];
-        }
+        for (int i = 0; i < 2; ++i) ra[i] = *(const uint4 *)(A + (m0 + lr + 32 * i) * H + k0 + lc);
 #pragma unroll
-        for (int j = 0; j < (BN * BK) / 256; ++j) {
-            int e = tid + 256 * j;
-            int nn, kk;
-            if (b_kfast) { nn = e / BK; kk = e % BK; } else { kk = e / BN; nn = e % BN; }
-            sB[nn][kk] = g.B[(long long)(k0 + kk) * g.sbk + (long long)(n0 + nn) * g.sbn];
-        }
+        for (int i = 0; i < 4; ++i) rb[i] = *(const uint4 *)(B + (size_t)(n0 + lr + 32 * i) * H + k0 + lc);
+    };
+    f32x16 acc[2];
+    for (int i = 0; i < 16; ++i) acc[0][i] = acc[1][i] = 0.f;
+    fetch(0);
+    const int r = lane & 31, kh = 4 * (lane >> 5);
+    for (int k0 = 0; k0 < H; k0 += GK) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) *(uint4 *)&sA[lr + 32 * i][lc] = ra[i];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) *(uint4 *)&sB[lr + 32 * i][lc] = rb[i];
         __syncthreads();
+        if (k0 + GK < H) fetch(k0 + GK);
 #pragma unroll
-        for (int kk = 0; kk < BK; kk += 8) {
-            // A fragment: row wm + lane%32, k = kk + 4*(lane/32) .. +3 ; B fragment: col wn + lane%32
-            const int r = lane & 31, kq = kk + 4 * (lane >> 5);
-            bf16x4 a, b;
-            for (int i = 0; i < 4; ++i) {
-                a[i] = (short)sA[wm + r][kq + i];
-                b[i] = (short)sB[wn + r][kq + i];
-            }
-            acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a, b, acc, 0, 0, 0);
+        for (int kk = 0; kk < GK; kk += 8) {
+            // A fragment: row wm + lane % 32, k = kk + 4 (lane / 32) .. + 3; B fragment: the same of its columns
+            const bf16x4 a = lds_frag(&sA[wm + r][kk + kh]);
+            acc[0] = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a, lds_frag(&sB[wn + r][kk + kh]), acc[0], 0, 0, 0);
+            acc[1] = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a, lds_frag(&sB[wn + 32 + r][kk + kh]), acc[1], 0, 0, 0);
         }
         __syncthreads();
     }
-    // accumulator element acc[4j+i]: row 8j + 4*(lane/32) + i, column lane % 32
-    const int col = n0 + wn + (lane & 31);
+    // accumulator element 4 j + i: row 8 j + 4 (lane / 32) + i, column lane % 32
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        const int col = n0 + wn + 32 * c + r;
+        const float bc = BWD ? 0.f : bias[col];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const size_t o = (m0 + wm + 8 * j + kh + i) * H + col;
+                const float v = acc[c][4 * j + i];
+                if (BWD) {
+                    out[o] = f2bf(v * silu_grad(Z[o]));
+                } else {
+                    const float z = v + bc;
+                    Z[o] = z;
+                    out[o] = f2bf(silu(z));
+                }
+            }
+    }
+}
+
+// Weight gradients of the three hidden layers, split over the batch: part[layer][split][n][k] = sum over the split's
+// rows of dZ[row][n] A[row][k].  Both operands are row-major over the summed index, so a thread loads a 4 x 4 block
+// (8 bytes of four rows) and stores it transposed.  Tile 64 x 64, blockIdx.z = layer * nsplit + split.
+struct WgradArgs {
+    const unsigned short *dZ[3], *A[3];
+};
+__global__ void __launch_bounds__(256) k_gemm_wgrad(WgradArgs g, int M, int kchunk, int nsplit, float *__restrict__ part)
+{
+    __shared__ __align__(16) unsigned short sA[64][GK + GPAD], sB[64][GK + GPAD];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int layer = blockIdx.z / nsplit, split = blockIdx.z - layer * nsplit;
+    const int m0 = blockIdx.x * 64, n0 = blockIdx.y * 64;
+    const int kbeg = split * kchunk, kend = min(M, kbeg + kchunk);
+    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+    const unsigned short *pa = g.dZ[layer] + m0, *pb = g.A[layer] + n0;
+    const int cg = (tid & 15) * 4, rg = (tid >> 4) * 4;  // this thread's block: columns cg.., rows rg.. of a stage
+    uint2 ra[4], rb[4];
+    auto fetch = [&](int k0) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int row = k0 + rg + i;
+            ra[i] = row < kend ? *(const uint2 *)(pa + (size_t)row * H + cg) : make_uint2(0u, 0u);
+            rb[i] = row < kend ? *(const uint2 *)(pb + (size_t)row * H + cg) : make_uint2(0u, 0u);
+        }
+    };
+    // column c of the block, rows 0..3, as one 8-byte store
+    auto put = [&](unsigned short(*sh)[GK + GPAD], const uint2 *v) {
+        auto lo = [](unsigned x, unsigned y) { return (x & 0xffffu) | (y << 16); };
+        auto hi = [](unsigned x, unsigned y) { return (x >> 16) | (y & 0xffff0000u); };
+        *(uint2 *)&sh[cg][rg] = make_uint2(lo(v[0].x, v[1].x), lo(v[2].x, v[3].x));
+        *(uint2 *)&sh[cg + 1][rg] = make_uint2(hi(v[0].x, v[1].x), hi(v[2].x, v[3].x));
+        *(uint2 *)&sh[cg + 2][rg] = make_uint2(lo(v[0].y, v[1].y), lo(v[2].y, v[3].y));
+        *(uint2 *)&sh[cg + 3][rg] = make_uint2(hi(v[0].y, v[1].y), hi(v[2].y, v[3].y));
+    };
+    f32x16 acc;
+    for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+    fetch(kbeg);
+    const int r = lane & 31, kh = 4 * (lane >> 5);
+    for (int k0 = kbeg; k0 < kend; k0 += GK) {
+        put(sA, ra);
+        put(sB, rb);
+        __syncthreads();
+        if (k0 + GK < kend) fetch(k0 + GK);
+#pragma unroll
+        for (int kk = 0; kk < GK; kk += 8)
+            acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(lds_frag(&sA[wm + r][kk + kh]), lds_frag(&sB[wn + r][kk + kh]),
+                                                           acc, 0, 0, 0);
+        __syncthreads();
+    }
+    float *C = part + (size_t)blockIdx.z * H * H;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int row = m0 + wm + 8 * j + 4 * (lane >> 5) + i;
-            float v = acc[4 * j + i];
-            if (g.epi == 0) {
-                g.C[((long long)blockIdx.z * g.M + row) * g.N + col] = v;
-            } else if (g.epi == 1) {
-                float z = v + g.bias[col];
-                g.Z[(long long)row * g.ldo + col] = z;
-                g.Aout[(long long)row * g.ldo + col] = f2bf(silu(z));
-            } else if (g.epi == 2) {
-                float z = g.Z[(long long)row * g.ldo + col];
-                g.Aout[(long long)row * g.ldo + col] = f2bf(v * silu_grad(z));
-            } else {
-                g.Aout[(long long)row * g.ldo + col] = f2bf(silu(v + g.bias[col]));
+        for (int i = 0; i < 4; ++i)
+            C[(size_t)(m0 + wm + 8 * j + kh + i) * H + n0 + wn + r] = acc[4 * j + i];
+}
+
+// the splits' sums, all three layers: G[W_l] = sum_z part[l][z]
+__global__ void k_reduce_parts(const float *__restrict__ part, int nz, float *__restrict__ G)
+{
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x, n = (size_t)H * H;
+    if (i >= n) return;
+    const int l = blockIdx.y;
+    const float *p = part + (size_t)l * nz * n + i;
+    float s = 0.f;
+    for (int z = 0; z < nz; ++z) s += p[(size_t)z * n];
+    G[(l == 0 ? OFF_W2 : l == 1 ? OFF_W3 : OFF_W4) + i] = s;
+}
+
+// Sums over the batch that are no GEMM: 8 columns per workgroup, a thread's rows are t, t + 256, ...  (16-byte loads);
+// then the wave's butterfly and the four waves in order.  blockIdx.y: 0..2 the bias gradients of the hidden layers
+// (column sums of dZ), 3 layer 1 (gW1[n][k] = sum_m dZ1[m][n] X[m][k], gb1[n] = sum_m dZ1[m][n]), 4 the output layer
+// (gW5[k] = sum_m dy[m] A4[m][k], and from the first workgroup gb5 = sum dy).
+struct SmallGradArgs {
+    const unsigned short *dZ[4];  // of layers 1..4
+    const unsigned short *A4;
+    const float *X, *dy;
+};
+template <int N>
+__device__ __forceinline__ void block_sums(float (&v)[N], float *out, int stride)
+{
+    __shared__ float red[4][N];
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+        for (int o = 32; o >= 1; o >>= 1) v[k] += __shfl_xor(v[k], o, 64);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0)
+        for (int k = 0; k < N; ++k) red[threadIdx.x >> 6][k] = v[k];
+    __syncthreads();
+    if (threadIdx.x < N)
+        out[threadIdx.x * stride] = red[0][threadIdx.x] + red[1][threadIdx.x] + red[2][threadIdx.x] + red[3][threadIdx.x];
+}
+__device__ __forceinline__ void load8(const unsigned short *p, float *f)
+{
+    const uint4 u = *(const uint4 *)p;
+    const unsigned w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        f[2 * i] = __uint_as_float(w[i] << 16);
+        f[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+    }
+}
+__global__ void __launch_bounds__(256) k_small_grads(SmallGradArgs g, int M, float *__restrict__ G)
+{
+    const int job = blockIdx.y, c0 = blockIdx.x * 8;
+    float f[8], s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (job < 3) {
+        const unsigned short *x = g.dZ[job + 1] + c0;
+        for (int m = threadIdx.x; m < M; m += 256) {
+            load8(x + (size_t)m * H, f);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) s[i] += f[i];
+        }
+        block_sums(s, G + OFF_B[job] + c0, 1);
+    } else if (job == 3) {
+        float w[8 * NIN];  // [unit][input]
+        for (int i = 0; i < 8 * NIN; ++i) w[i] = 0.f;
+        for (int m = threadIdx.x; m < M; m += 256) {
+            load8(g.dZ[0] + (size_t)m * H + c0, f);
+            float x[NIN];
+#pragma unroll
+            for (int k = 0; k < NIN; ++k) x[k] = g.X[(size_t)m * NIN + k];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+#pragma unroll
+                for (int k = 0; k < NIN; ++k) w[i * NIN + k] += f[i] * x[k];
+                s[i] += f[i];
             }
         }
-}
-
-// sum of split-K partials: out[i] = sum_z part[z][i]
-__global__ void k_reduce_parts(const float *part, int nz, size_t n, float *out)
-{
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float s = 0.f;
-    for (int z = 0; z < nz; ++z) s += part[(size_t)z * n + i];
-    out[i] = s;
-}
-
-// column sums of a BF16 [M][N] matrix (bias gradients): out[n] = sum_m X[m][n]
-__global__ void k_colsum_bf16(const unsigned short *X, int M, int N, float *out)
-{
-    int n = blockIdx.x;
-    float s = 0.f;
-    for (int m = threadIdx.x; m < M; m += blockDim.x) s += bf2f(X[(size_t)m * N + n]);
-    for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
-    __shared__ float red[4];
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) out[n] = red[0] + red[1] + red[2] + red[3];
+        block_sums(w, G + OFF_W1 + c0 * NIN, 1);
+        block_sums(s, G + OFF_B1 + c0, 1);
+    } else {
+        float b[1] = {0.f};
+        for (int m = threadIdx.x; m < M; m += 256) {
+            load8(g.A4 + (size_t)m * H + c0, f);
+            const float d = g.dy[m];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) s[i] += d * f[i];
+            b[0] += d;
+        }
+        block_sums(s, G + OFF_W5 + c0, 1);
+        if (blockIdx.x == 0) block_sums(b, G + OFF_B5, 1);
+    }
 }
 
 // layer 1 forward: Z1 = X W1^T + b1 (FP32), A1 = bf16(silu(Z1)); one thread per (row, unit)
@@ -201,68 +309,45 @@ __global__ void k_layer1_fwd(const float *X, int M, const float *P, float *Z1, u
     A1[t] = f2bf(silu(z));
 }
 
-// output layer forward: y = A4 w5 + b5 (one wave per row); optional loss gradient and dZ4
+// output layer forward: y = A4 w5 + b5, kOutRows rows per wave, one after the other; optional loss gradient and dZ4.
+// The loss takes one atomic per workgroup: one per row serialised on its address (8192 rows 104 us).
+constexpr int kOutRows = 4;
 __global__ void __launch_bounds__(256) k_out_fwd(const unsigned short *A4, const float *Z4, int M, const float *P,
                                                  float *y, const float *target, float inv_batch, float *dy,
                                                  unsigned short *dZ4, double *loss)
 {
-    int wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, lane = threadIdx.x & 63;
-    if (wave >= M) return;
-    const unsigned short *a = A4 + (size_t)wave * H;
-    float s = 0.f;
-    for (int k = lane; k < H; k += 64) s += bf2f(a[k]) * P[OFF_W5 + k];
-    for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
-    float yy = s + P[OFF_B5];
-    if (lane == 0 && y) y[wave] = yy;
-    if (target) {
-        float d = (yy - target[wave]) * inv_batch;  // d/dy of mean (y-t)^2/2
-        if (lane == 0) {
-            dy[wave] = d;
-            atomicAdd(loss, 0.5 * (double)(yy - target[wave]) * (double)(yy - target[wave]) * inv_batch);
+    __shared__ double red[4];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int row0 = (blockIdx.x * 4 + wv) * kOutRows;
+    float w[H / 64];
+#pragma unroll
+    for (int j = 0; j < H / 64; ++j) w[j] = P[OFF_W5 + lane + 64 * j];
+    const float b5 = P[OFF_B5];
+    double sum = 0;
+    for (int row = row0; row < min(M, row0 + kOutRows); ++row) {
+        const unsigned short *a = A4 + (size_t)row * H;
+        float s = 0.f;
+#pragma unroll
+        for (int j = 0; j < H / 64; ++j) s += bf2f(a[lane + 64 * j]) * w[j];
+        for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
+        float yy = s + b5;
+        if (lane == 0 && y) y[row] = yy;
+        if (target) {
+            const float t = target[row];
+            float d = (yy - t) * inv_batch;  // d/dy of mean (y-t)^2/2
+            if (lane == 0) dy[row] = d;
+            sum += 0.5 * (double)(yy - t) * (double)(yy - t) * inv_batch;
+#pragma unroll
+            for (int j = 0; j < H / 64; ++j) {
+                const size_t o = (size_t)row * H + lane + 64 * j;
+                dZ4[o] = f2bf(d * w[j] * silu_grad(Z4[o]));
+            }
         }
-        for (int k = lane; k < H; k += 64) {
-            float z = Z4[(size_t)wave * H + k];
-            dZ4[(size_t)wave * H + k] = f2bf(d * P[OFF_W5 + k] * silu_grad(z));
-        }
     }
-}
-
-// output-layer gradients: gW5[k] = sum_m dy[m] A4[m][k], gb5 = sum dy
-__global__ void k_out_grad(const unsigned short *A4, const float *dy, int M, float *G)
-{
-    int k = blockIdx.x;  // 0..H (H -> bias)
-    float s = 0.f;
-    for (int m = threadIdx.x; m < M; m += blockDim.x) s += dy[m] * (k < H ? bf2f(A4[(size_t)m * H + k]) : 1.0f);
-    for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
-    __shared__ float red[4];
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    if (!target) return;  // every thread alike
+    if (lane == 0) red[wv] = sum;
     __syncthreads();
-    if (threadIdx.x == 0) G[k < H ? OFF_W5 + k : OFF_B5] = red[0] + red[1] + red[2] + red[3];
-}
-
-// layer-1 gradients: gW1[n][k] = sum_m dZ1[m][n] X[m][k], gb1[n] = sum_m dZ1[m][n]
-__global__ void k_layer1_grad(const unsigned short *dZ1, const float *X, int M, float *G)
-{
-    int n = blockIdx.x;
-    float s[NIN + 1];
-    for (int k = 0; k <= NIN; ++k) s[k] = 0.f;
-    for (int m = threadIdx.x; m < M; m += blockDim.x) {
-        float d = bf2f(dZ1[(size_t)m * H + n]);
-        for (int k = 0; k < NIN; ++k) s[k] += d * X[(size_t)m * NIN + k];
-        s[NIN] += d;
-    }
-    __shared__ float red[NIN + 1][4];
-    for (int k = 0; k <= NIN; ++k) {
-        float v = s[k];
-        for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-        if ((threadIdx.x & 63) == 0) red[k][threadIdx.x >> 6] = v;
-    }
-    __syncthreads();
-    if (threadIdx.x <= NIN) {
-        float v = red[threadIdx.x][0] + red[threadIdx.x][1] + red[threadIdx.x][2] + red[threadIdx.x][3];
-        if (threadIdx.x < NIN) G[OFF_W1 + n * NIN + threadIdx.x] = v;
-        else G[OFF_B1 + n] = v;
-    }
+    if (threadIdx.x == 0) atomicAdd(loss, red[0] + red[1] + red[2] + red[3]);
 }
 
 __global__ void k_adam(float *P, const float *G, float *m, float *v, size_t n, float lr, float b1, float b2, float eps,
@@ -278,7 +363,7 @@ __global__ void k_adam(float *P, const float *G, float *m, float *v, size_t n, f
     P[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
 }
 
-// FP32 -> BF16 copies of W2..W4 ([out][in] row-major)
+// FP32 -> BF16 copies of W2..W4: [out][in], and behind the three of them [in][out] for the backward products
 __global__ void k_weights_bf16(const float *P, unsigned short *Wb)
 {
     size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -286,7 +371,9 @@ __global__ void k_weights_bf16(const float *P, unsigned short *Wb)
     int l = (int)(t / (H * H));
     size_t e = t % (H * H);
     const size_t off[3] = {OFF_W2, OFF_W3, OFF_W4};
-    Wb[t] = f2bf(P[off[l] + e]);
+    const unsigned short w = f2bf(P[off[l] + e]);
+    Wb[t] = w;
+    Wb[(size_t)(NLAYER_MFMA + l) * H * H + (e % H) * H + e / H] = w;
 }
 
 // --------------------------------------------------------------- data generation
@@ -416,7 +503,7 @@ struct TpSurRoundBufs {
 struct TpSurrogate {
     TpSurRoundBufs rb[TP_NLANES];
     float *P = nullptr, *G = nullptr, *Am = nullptr, *Av = nullptr;
-    unsigned short *Wb = nullptr;  // [3][H][H]
+    unsigned short *Wb = nullptr;  // [3][H][H] W2..W4, then their transposes
     uint4 *Wf = nullptr;           // [NFRAG] hidden weights, BF16, in k_mlp_reg's fragment order
     uint4 *Wh = nullptr;           // [NFRAG] the same BF16 weights as FP16 (exact), for k_mlp_h
     int infer = TP_SUR_INFER_FP16; // inference kernel (tp_surrogate_inference)
@@ -441,7 +528,7 @@ static int sur_alloc(TpSurrogate *s)
     TP_HIP(hipMalloc(&s->G, NPARAM * sizeof(float)));
     TP_HIP(hipMalloc(&s->Am, NPARAM * sizeof(float)));
     TP_HIP(hipMalloc(&s->Av, NPARAM * sizeof(float)));
-    TP_HIP(hipMalloc(&s->Wb, 3 * H * H * sizeof(unsigned short)));
+    TP_HIP(hipMalloc(&s->Wb, 2 * 3 * H * H * sizeof(unsigned short)));
     TP_HIP(hipMalloc(&s->Wf, NFRAG * sizeof(uint4)));
     TP_HIP(hipMalloc(&s->Wh, NFRAG * sizeof(uint4)));
     TP_HIP(hipMalloc(&s->d_loss, sizeof(double)));
@@ -468,7 +555,7 @@ static int sur_ensure_batch(TpSurrogate *s, int rows)
         TP_HIP(hipMalloc(&s->dZ[i], (size_t)cap * H * sizeof(unsigned short)));
     }
     s->nsplit = std::max(1, std::min(64, cap / 256));
-    TP_HIP(hipMalloc(&s->parts, (size_t)s->nsplit * H * H * sizeof(float)));
+    TP_HIP(hipMalloc(&s->parts, (size_t)3 * s->nsplit * H * H * sizeof(float)));
     s->cap = cap;
     return 0;
 }
@@ -492,38 +579,16 @@ void tp_surrogate_free(tp_ctx *ctx)
     }
 }
 
-static void launch_gemm(hipStream_t st, const GemmArgs &g, int nsplit)
-{
-    dim3 gr(g.M / BM, g.N / BN, nsplit);
-    hipLaunchKernelGGL(k_gemm_bf16, gr, dim3(256), 0, st, g);
-}
-
 // forward over rows [0, M) of s->X (M % 64 == 0); leaves Y (standardised log B)
 static int sur_forward(hipStream_t st, TpSurrogate *s, int M, const float *target, double *loss_accum)
 {
     hipLaunchKernelGGL(k_layer1_fwd, dim3(grid((size_t)M * H, 256)), dim3(256), 0, st, s->X, M, s->P, s->Z[0],
                        s->A[0]);
-    for (int l = 0; l < 3; ++l) {
-        GemmArgs g{};
-        g.A = s->A[l];
-        g.sam = H;
-        g.sak = 1;
-        g.B = s->Wb + (size_t)l * H * H;  // B(k, n) = W[n][k]
-        g.sbk = 1;
-        g.sbn = H;
-        g.M = M;
-        g.N = H;
-        g.K = H;
-        g.kchunk = H;
-        g.epi = 1;
-        g.bias = s->P + OFF_B[l];
-        g.Z = s->Z[l + 1];
-        g.Aout = s->A[l + 1];
-        g.ldo = H;
-        launch_gemm(st, g, 1);
-    }
-    hipLaunchKernelGGL(k_out_fwd, dim3(grid((size_t)M * 64, 256)), dim3(256), 0, st, s->A[3], s->Z[3], M, s->P, s->Y,
-                       target, 1.0f / (float)M, s->dy, s->dZ[3], loss_accum);
+    for (int l = 0; l < 3; ++l)
+        hipLaunchKernelGGL(k_gemm_rows<false>, dim3(M / GM, H / GN), dim3(256), 0, st, s->A[l],
+                           s->Wb + (size_t)l * H * H, s->P + OFF_B[l], s->Z[l + 1], s->A[l + 1]);
+    hipLaunchKernelGGL(k_out_fwd, dim3(grid(M, 4 * kOutRows)), dim3(256), 0, st, s->A[3], s->Z[3], M, s->P, s->Y, target,
+                       1.0f / (float)M, s->dy, s->dZ[3], loss_accum);
     TP_HIP(hipGetLastError());
     return 0;
 }
@@ -531,48 +596,28 @@ static int sur_forward(hipStream_t st, TpSurrogate *s, int M, const float *targe
 // backward after sur_forward with a target: gradients into s->G
 static int sur_backward(hipStream_t st, TpSurrogate *s, int M)
 {
-    hipLaunchKernelGGL(k_out_grad, dim3(H + 1), dim3(256), 0, st, s->A[3], s->dy, M, s->G);
-    for (int l = 2; l >= 0; --l) {
-        // weight gradient: gW[n][k] = sum_m dZ[l+1][m][n] A[l][m][k]  (split-K over the batch)
-        GemmArgs g{};
-        g.A = s->dZ[l + 1];
-        g.sam = 1;
-        g.sak = H;  // A(m=n_out, k=row) = dZ[row][n_out]
-        g.B = s->A[l];
-        g.sbk = H;
-        g.sbn = 1;  // B(k=row, n=k_in) = A[row][k_in]
-        g.M = H;
-        g.N = H;
-        g.K = M;
-        int ns = std::max(1, std::min(s->nsplit, M / BK));
-        int kc = ((M / ns + BK - 1) / BK) * BK;
-        ns = (M + kc - 1) / kc;
-        g.kchunk = kc;
-        g.epi = 0;
-        g.C = s->parts;
-        launch_gemm(st, g, ns);
-        hipLaunchKernelGGL(k_reduce_parts, dim3(grid((size_t)H * H, 256)), dim3(256), 0, st, s->parts, ns,
-                           (size_t)H * H, s->G + OFF_W[l]);
-        hipLaunchKernelGGL(k_colsum_bf16, dim3(H), dim3(256), 0, st, s->dZ[l + 1], M, H, s->G + OFF_B[l]);
-        // input gradient: dZ[l][m][k] = (sum_n dZ[l+1][m][n] W[n][k]) * silu'(Z[l][m][k])
-        GemmArgs h{};
-        h.A = s->dZ[l + 1];
-        h.sam = H;
-        h.sak = 1;
-        h.B = s->Wb + (size_t)l * H * H;  // B(k=n_out, n=k_in) = W[n_out][k_in]
-        h.sbk = H;
-        h.sbn = 1;
-        h.M = M;
-        h.N = H;
-        h.K = H;
-        h.kchunk = H;
-        h.epi = 2;
-        h.Z = s->Z[l];
-        h.Aout = s->dZ[l];
-        h.ldo = H;
-        launch_gemm(st, h, 1);
+    // dZ of layers 3, 2, 1: dZ[l] = (dZ[l + 1] W) SiLU'(Z[l])
+    for (int l = 2; l >= 0; --l)
+        hipLaunchKernelGGL(k_gemm_rows<true>, dim3(M / GM, H / GN), dim3(256), 0, st, s->dZ[l + 1],
+                           s->Wb + (size_t)(NLAYER_MFMA + l) * H * H, (const float *)nullptr, s->Z[l], s->dZ[l]);
+    // then every gradient: the weights' (split over the batch) and the sums
+    constexpr int kc0 = 32;  // splits are whole multiples of this many rows
+    int ns = std::max(1, std::min(s->nsplit, M / kc0));
+    const int kc = ((M / ns + kc0 - 1) / kc0) * kc0;
+    ns = (M + kc - 1) / kc;
+    WgradArgs wa{};
+    SmallGradArgs sa{};
+    for (int l = 0; l < 3; ++l) {
+        wa.dZ[l] = s->dZ[l + 1];
+        wa.A[l] = s->A[l];
     }
-    hipLaunchKernelGGL(k_layer1_grad, dim3(H), dim3(256), 0, st, s->dZ[0], s->X, M, s->G);
+    for (int l = 0; l < 4; ++l) sa.dZ[l] = s->dZ[l];
+    sa.A4 = s->A[3];
+    sa.X = s->X;
+    sa.dy = s->dy;
+    hipLaunchKernelGGL(k_gemm_wgrad, dim3(H / 64, H / 64, 3 * ns), dim3(256), 0, st, wa, M, kc, ns, s->parts);
+    hipLaunchKernelGGL(k_small_grads, dim3(H / 8, 5), dim3(256), 0, st, sa, M, s->G);
+    hipLaunchKernelGGL(k_reduce_parts, dim3(H * H / 256, 3), dim3(256), 0, st, s->parts, ns, s->G);
     TP_HIP(hipGetLastError());
     return 0;
 }
