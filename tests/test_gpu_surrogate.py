@@ -246,3 +246,11 @@ def test_surrogate_form_within_1e3_of_fp64(gpu_ctx, fid_nz, workload):
     assert err.max() <= 1e-3
     # the network serves what the exact rules leave: ~60% of C1's points, ~47% of the C3 subset's
     assert st["surrogate_points"] > 0.4 * st["points"]
+
+
+@pytest.mark.parametrize("M", [192, 4160])
+def test_mlp_gradients_of_ragged_batches(gpu_ctx, M):
+    """Batches whose weight-gradient splits end inside a 64-row stage (192 rows: splits of 192; 4160: 16 splits of 288
+    rows and a last one that is shorter) and whose column sums have a partial last pass, against the oracle at the
+    tolerance of test_mlp_gradients_match_cpu_oracle."""
+    test_mlp_gradients_match_cpu_oracle(gpu_ctx, M)

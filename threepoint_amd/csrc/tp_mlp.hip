@@ -81,13 +81,14 @@ constexpr size_t OFF_B[3] = {OFF_B2, OFF_B3, OFF_B4};
 // The hidden layers of a training batch, BF16 operands with FP32 accumulation by 32x32x8 MFMAs, K ascending.  A batch of
 // 8192 rows is 1 GFLOP per product, a microsecond of matrix-core time: what counts is that operands arrive in 16-byte
 // loads, that the next stage's are in flight during the MFMAs, and how many launches a step takes (8192 rows forward and
-// backward: 577 us on the device with 2-byte loads, one launch per gradient and an atomic per row for the loss; @MLP@
-// in this form, gradients unchanged to the bit).
-constexpr int GM = 64, GN = 128, GK = 64, GPAD = 8;
+// backward: 577 us on the device with 2-byte loads, one launch per gradient and an atomic per row for the loss; 165 us
+// in this form, gradients unchanged to the bit).  Per product 30-38 -> 13-15 us; 128 columns a tile: 18-23 us, one workgroup
+// per CU.
+constexpr int GM = 64, GN = 64, GK = 64, GPAD = 8;
 
 __device__ __forceinline__ bf16x4 lds_frag(const unsigned short *p) { return *(const bf16x4 *)p; }
 
-// C[M][H] = sum_k A(m, k) B(n, k), both k-contiguous with row length H.  Tile 64 x 128, four waves of 32 x 64.
+// C[M][H] = sum_k A(m, k) B(n, k), both k-contiguous with row length H.  Tile 64 x 64, four waves of 32 x 32.
 // BWD false: Z = C + bias, out = bf16(SiLU(Z)).  BWD true: out = bf16(C SiLU'(Z)).  M % 64 == 0 (checked on the host).
 template <bool BWD>
 __global__ void __launch_bounds__(256) k_gemm_rows(const unsigned short *__restrict__ A,
@@ -98,54 +99,52 @@ __global__ void __launch_bounds__(256) k_gemm_rows(const unsigned short *__restr
     __shared__ __align__(16) unsigned short sA[GM][GK + GPAD], sB[GN][GK + GPAD];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const size_t m0 = (size_t)blockIdx.x * GM;
-    const int n0 = blockIdx.y * GN, wm = (wave >> 1) * 32, wn = (wave & 1) * 64;
+    const int n0 = blockIdx.y * GN, wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
     const int lr = tid >> 3, lc = (tid & 7) * 8;  // this thread's row (of 32 per load) and first k
-    uint4 ra[2], rb[4];
+    uint4 ra[2], rb[2];
     auto fetch = [&](int k0) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) ra[i] = *(const uint4 *)(A + (m0 + lr + 32 * i) * H + k0 + lc);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) rb[i] = *(const uint4 *)(B + (size_t)(n0 + lr + 32 * i) * H + k0 + lc);
+        for (int i = 0; i < 2; ++i) rb[i] = *(const uint4 *)(B + (size_t)(n0 + lr + 32 * i) * H + k0 + lc);
     };
-    f32x16 acc[2];
-    for (int i = 0; i < 16; ++i) acc[0][i] = acc[1][i] = 0.f;
+    f32x16 acc;
+    for (int i = 0; i < 16; ++i) acc[i] = 0.f;
     fetch(0);
     const int r = lane & 31, kh = 4 * (lane >> 5);
     for (int k0 = 0; k0 < H; k0 += GK) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) *(uint4 *)&sA[lr + 32 * i][lc] = ra[i];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) *(uint4 *)&sB[lr + 32 * i][lc] = rb[i];
+        for (int i = 0; i < 2; ++i) *(uint4 *)&sB[lr + 32 * i][lc] = rb[i];
         __syncthreads();
         if (k0 + GK < H) fetch(k0 + GK);
 #pragma unroll
-        for (int kk = 0; kk < GK; kk += 8) {
+        for (int kk = 0; kk < GK; kk += 8)
             // A fragment: row wm + lane % 32, k = kk + 4 (lane / 32) .. + 3; B fragment: the same of its columns
-            const bf16x4 a = lds_frag(&sA[wm + r][kk + kh]);
-            acc[0] = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a, lds_frag(&sB[wn + r][kk + kh]), acc[0], 0, 0, 0);
-            acc[1] = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a, lds_frag(&sB[wn + 32 + r][kk + kh]), acc[1], 0, 0, 0);
-        }
+            acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(lds_frag(&sA[wm + r][kk + kh]), lds_frag(&sB[wn + r][kk + kh]),
+                                                           acc, 0, 0, 0);
         __syncthreads();
     }
     // accumulator element 4 j + i: row 8 j + 4 (lane / 32) + i, column lane % 32
+    const int col = n0 + wn + r;
+    const float bc = BWD ? 0.f : bias[col];
+    const size_t o0 = (m0 + wm + kh) * H + col;
+    float z[16];
+    if (BWD) {
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-        const int col = n0 + wn + 32 * c + r;
-        const float bc = BWD ? 0.f : bias[col];
+        for (int e = 0; e < 16; ++e) z[e] = Z[o0 + (size_t)(8 * (e >> 2) + (e & 3)) * H];
+    }
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const size_t o = (m0 + wm + 8 * j + kh + i) * H + col;
-                const float v = acc[c][4 * j + i];
-                if (BWD) {
-                    out[o] = f2bf(v * silu_grad(Z[o]));
-                } else {
-                    const float z = v + bc;
-                    Z[o] = z;
-                    out[o] = f2bf(silu(z));
-                }
-            }
+    for (int e = 0; e < 16; ++e) {
+        const size_t o = o0 + (size_t)(8 * (e >> 2) + (e & 3)) * H;
+        if (BWD) {
+            out[o] = f2bf(acc[e] * silu_grad(z[e]));
+        } else {
+            const float zz = acc[e] + bc;
+            Z[o] = zz;
+            out[o] = f2bf(silu(zz));
+        }
     }
 }
 
@@ -218,10 +217,11 @@ __global__ void k_reduce_parts(const float *__restrict__ part, int nz, float *__
     G[(l == 0 ? OFF_W2 : l == 1 ? OFF_W3 : OFF_W4) + i] = s;
 }
 
-// Sums over the batch that are no GEMM: 8 columns per workgroup, a thread's rows are t, t + 256, ...  (16-byte loads);
-// then the wave's butterfly and the four waves in order.  blockIdx.y: 0..2 the bias gradients of the hidden layers
-// (column sums of dZ), 3 layer 1 (gW1[n][k] = sum_m dZ1[m][n] X[m][k], gb1[n] = sum_m dZ1[m][n]), 4 the output layer
-// (gW5[k] = sum_m dy[m] A4[m][k], and from the first workgroup gb5 = sum dy).
+// Sums over the batch that are no GEMM: a thread's rows are t, t + 256, ... (16-byte loads), then the wave's butterfly and
+// the four waves in order.  A workgroup takes 16 columns (8 units of layer 1): with 4 each, the rows' cache lines went
+// through the L2 64 times, 34 us for 8192 rows, now 25.  Jobs: 0..2 the bias gradients of the hidden layers (column sums
+// of dZ), 3 the output layer (gW5[k] = sum_m dy[m] A4[m][k], its first workgroup gb5 = sum dy), 4 and 5 layer 1
+// (gW1[n][k] = sum_m dZ1[m][n] X[m][k], gb1[n] = sum_m dZ1[m][n]).
 struct SmallGradArgs {
     const unsigned short *dZ[4];  // of layers 1..4
     const unsigned short *A4;
@@ -251,47 +251,61 @@ __device__ __forceinline__ void load8(const unsigned short *p, float *f)
         f[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
     }
 }
+constexpr int kSumCols = 16, kSumUnits = 8, kSumBlocks = H / kSumCols;
+static_assert(2 * kSumBlocks * kSumUnits == H, "jobs 4 and 5 cover layer 1");
 __global__ void __launch_bounds__(256) k_small_grads(SmallGradArgs g, int M, float *__restrict__ G)
 {
-    const int job = blockIdx.y, c0 = blockIdx.x * 8;
-    float f[8], s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (job < 3) {
-        const unsigned short *x = g.dZ[job + 1] + c0;
-        for (int m = threadIdx.x; m < M; m += 256) {
-            load8(x + (size_t)m * H, f);
+    const int job = blockIdx.y;
+    if (job < 4) {
+        const int c0 = blockIdx.x * kSumCols;
+        const unsigned short *x = (job < 3 ? g.dZ[job + 1] : g.A4) + c0;
+        float f[kSumCols], s[kSumCols], b[1] = {0.f};
 #pragma unroll
-            for (int i = 0; i < 8; ++i) s[i] += f[i];
-        }
-        block_sums(s, G + OFF_B[job] + c0, 1);
-    } else if (job == 3) {
-        float w[8 * NIN];  // [unit][input]
-        for (int i = 0; i < 8 * NIN; ++i) w[i] = 0.f;
-        for (int m = threadIdx.x; m < M; m += 256) {
-            load8(g.dZ[0] + (size_t)m * H + c0, f);
-            float x[NIN];
+        for (int i = 0; i < kSumCols; ++i) s[i] = 0.f;
+        if (job < 3) {
+#pragma unroll 4
+            for (int m = threadIdx.x; m < M; m += 256) {
+                load8(x + (size_t)m * H, f);
+                load8(x + (size_t)m * H + 8, f + 8);
 #pragma unroll
-            for (int k = 0; k < NIN; ++k) x[k] = g.X[(size_t)m * NIN + k];
+                for (int i = 0; i < kSumCols; ++i) s[i] += f[i];
+            }
+        } else {
+#pragma unroll 4
+            for (int m = threadIdx.x; m < M; m += 256) {
+                load8(x + (size_t)m * H, f);
+                load8(x + (size_t)m * H + 8, f + 8);
+                const float d = g.dy[m];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-#pragma unroll
-                for (int k = 0; k < NIN; ++k) w[i * NIN + k] += f[i] * x[k];
-                s[i] += f[i];
+                for (int i = 0; i < kSumCols; ++i) s[i] += d * f[i];
+                b[0] += d;
             }
         }
-        block_sums(w, G + OFF_W1 + c0 * NIN, 1);
-        block_sums(s, G + OFF_B1 + c0, 1);
-    } else {
-        float b[1] = {0.f};
-        for (int m = threadIdx.x; m < M; m += 256) {
-            load8(g.A4 + (size_t)m * H + c0, f);
-            const float d = g.dy[m];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) s[i] += d * f[i];
-            b[0] += d;
-        }
-        block_sums(s, G + OFF_W5 + c0, 1);
-        if (blockIdx.x == 0) block_sums(b, G + OFF_B5, 1);
+        block_sums(s, G + (job < 3 ? OFF_B[job] : OFF_W5) + c0, 1);
+        if (job == 3 && blockIdx.x == 0) block_sums(b, G + OFF_B5, 1);
+        return;
     }
+    const int c0 = ((job - 4) * kSumBlocks + blockIdx.x) * kSumUnits;
+    float f[kSumUnits], s[kSumUnits], w[kSumUnits * NIN];  // w: [unit][input]
+#pragma unroll
+    for (int i = 0; i < kSumUnits; ++i) s[i] = 0.f;
+#pragma unroll
+    for (int i = 0; i < kSumUnits * NIN; ++i) w[i] = 0.f;
+#pragma unroll 2
+    for (int m = threadIdx.x; m < M; m += 256) {
+        load8(g.dZ[0] + (size_t)m * H + c0, f);
+        float x[NIN];
+#pragma unroll
+        for (int k = 0; k < NIN; ++k) x[k] = g.X[(size_t)m * NIN + k];
+#pragma unroll
+        for (int i = 0; i < kSumUnits; ++i) {
+#pragma unroll
+            for (int k = 0; k < NIN; ++k) w[i * NIN + k] += f[i] * x[k];
+            s[i] += f[i];
+        }
+    }
+    block_sums(w, G + OFF_W1 + c0 * NIN, 1);
+    block_sums(s, G + OFF_B1 + c0, 1);
 }
 
 // layer 1 forward: Z1 = X W1^T + b1 (FP32), A1 = bf16(silu(Z1)); one thread per (row, unit)
@@ -616,7 +630,7 @@ static int sur_backward(hipStream_t st, TpSurrogate *s, int M)
     sa.X = s->X;
     sa.dy = s->dy;
     hipLaunchKernelGGL(k_gemm_wgrad, dim3(H / 64, H / 64, 3 * ns), dim3(256), 0, st, wa, M, kc, ns, s->parts);
-    hipLaunchKernelGGL(k_small_grads, dim3(H / 8, 5), dim3(256), 0, st, sa, M, s->G);
+    hipLaunchKernelGGL(k_small_grads, dim3(kSumBlocks, 6), dim3(256), 0, st, sa, M, s->G);
     hipLaunchKernelGGL(k_reduce_parts, dim3(H * H / 256, 3), dim3(256), 0, st, s->parts, ns, s->G);
     TP_HIP(hipGetLastError());
     return 0;
