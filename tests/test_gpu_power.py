@@ -117,6 +117,42 @@ def test_power_with_tabulated_pk(gpu_ctx, fid_nz):
         assert n[i] == on and abs(v[i] / ov - 1) < 1e-10
 
 
+@pytest.mark.parametrize("n", [16, 40, 1100])
+@pytest.mark.parametrize("flags,sigma,reltol", [(0, 0.0, 1e-5), (tp.PK_T17, 0.3, 5e-6), (tp.PK_LINEAR, 0.0, 1e-3)])
+def test_map2_batch_sizes_agree(fid_tables, n, flags, sigma, reltol):
+    """Integrals finished on the device, in either workgroup size, and in rounds take the same steps in the same
+    order: equal bits."""
+    th = np.geomspace(0.3, 100, n) * A
+    v, e, m = fid_tables.map2_batch(th, reltol=reltol, flags=flags, sigma=sigma, ngal=30.0)
+    pick = np.unique(np.linspace(0, n - 1, 45).astype(int))
+    for c in np.array_split(pick, 4):  # fewer than 16 to a call
+        rv, re, rm = fid_tables.map2_batch(th[c], reltol=reltol, flags=flags, sigma=sigma, ngal=30.0)
+        assert np.array_equal(v[c], rv) and np.array_equal(e[c], re) and np.array_equal(m[c], rm)
+
+
+@pytest.mark.parametrize("reltol", [5e-6, 5e-5])
+def test_map2_integrals_that_outgrow_the_device(gpu_ctx, fid_nz, reltol):
+    """A coarsely tabulated P(k) has kinks: integrals that hold more regions than the device keeps of one (all of
+    them at the tighter tolerance) are finished in rounds, with the bits of calls in rounds; a round limit ends the
+    call."""
+    kh = np.geomspace(1e-4, 50, 12)
+    tabs = tp.CosmologyTables([W.fiducial()], fid_nz, 100, 3.0, gpu_ctx, pk=(kh, 2e4 * (kh / 0.02) / (1 + (kh / 0.02) ** 2.5)))
+    th = np.geomspace(0.5, 64, 28) * A
+    v, e, m = tabs.map2_batch(th, reltol=reltol, flags=tp.PK_LINEAR)
+    held = (m // 17 + 1) // 2
+    print("regions held: %d to %d" % (held.min(), held.max()))
+    assert held.max() > 1024 or reltol > 5e-6
+    for c in (slice(0, 14), slice(14, 28)):
+        rv, re, rm = tabs.map2_batch(th[c], reltol=reltol, flags=tp.PK_LINEAR)
+        assert np.array_equal(v[c], rv) and np.array_equal(e[c], re) and np.array_equal(m[c], rm)
+    gpu_ctx.set_batch_limits(max_rounds=3)
+    try:
+        with pytest.raises(tp.TpError, match=r"code 4\).*round limit"):
+            tabs.map2_batch(th, reltol=1e-5)
+    finally:
+        gpu_ctx.set_batch_limits()
+
+
 def test_power_rejects_bad_arguments(fid_tables):
     with pytest.raises(tp.TpError):
         fid_tables.map2_batch(np.array([0.0]))

@@ -377,16 +377,11 @@ __global__ void __launch_bounds__(256) k_map2_region_points(const TpCosmoConst *
                                  D.sigma, D.ngal);
 }
 
-// One thread per region: value, error and split axis from its 17 values, in the arithmetic order of
-// the host rule (classed_version/hcubature.cpp:515-575 with dim = 2, fdim = 1), contraction off.
-__global__ void __launch_bounds__(256) k_map2_region_rule(size_t nreg, const TpRegion2 *__restrict__ reg,
-                                                          const double *__restrict__ fv,
-                                                          TpRegion2Out *__restrict__ out)
+// Value, error and split axis of a region from its 17 values, in the arithmetic order of the host rule
+// (classed_version/hcubature.cpp:515-575 with dim = 2, fdim = 1), contraction off.
+__device__ __forceinline__ TpRegion2Out gm_rule2(double vol, const double *v)
 {
 #pragma clang fp contract(off)
-    const size_t r = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nreg) return;
-    const double *v = fv + r * kGm2Pts;
     const double l2 = 0.3585685828003180919906451539079374954541;  // sqrt(9/70)
     const double l4 = 0.9486832980505137995996680633298155601160;  // sqrt(9/10)
     const double ratio = (l2 * l2) / (l4 * l4);
@@ -406,7 +401,6 @@ __global__ void __launch_bounds__(256) k_map2_region_rule(size_t nreg, const TpR
     }
     for (int k = 0; k < 4; ++k) sum4 += v[9 + k];
     for (int k = 0; k < 4; ++k) sum5 += v[13 + k];
-    const double vol = reg[r].vol;
     const double result = vol * (w1 * val0 + wt2 * sum2 + w3 * sum3 + wt4 * sum4 + w5 * sum5);
     const double res5th = vol * (wE1 * val0 + wtE2 * sum2 + wE3 * sum3 + wtE4 * sum4);
     TpRegion2Out o;
@@ -420,7 +414,216 @@ __global__ void __launch_bounds__(256) k_map2_region_rule(size_t nreg, const TpR
             o.split = i;
         }
     o.flag = (isfinite(result) && isfinite(res5th)) ? 0 : 1;
-    out[r] = o;
+    return o;
+}
+
+// One thread per region: the rule.
+__global__ void __launch_bounds__(256) k_map2_region_rule(size_t nreg, const TpRegion2 *__restrict__ reg,
+                                                          const double *__restrict__ fv,
+                                                          TpRegion2Out *__restrict__ out)
+{
+    const size_t r = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (r < nreg) out[r] = gm_rule2(reg[r].vol, fv + r * kGm2Pts);
+}
+
+constexpr int kMap2Regions = 1024;  // regions an integral may hold on the device (~700 at a tolerance of 1e-5)
+constexpr int kMap2Chunk = 60;  // regions whose points are in LDS together (1020)
+struct TpMap2Region {
+    double c[2], hw[2], vol, val;
+    int split, pad;
+};
+struct TpMap2Out {
+    double val, err;
+    long long nreg;  // regions evaluated
+    int rounds;
+    int host;  // nonzero: not finished here (too many regions or rounds, a value not finite)
+};
+
+// A whole integral per workgroup, which takes integrals from a queue: the regions in its pool (global memory, in its
+// XCD's L2), the heap of their errors in LDS.  Points, rule and cuts are spread over the threads; the heap, and the sums
+// of value and error that decide, are thread 0's, in the order and arithmetic of tpc::AdaptiveIntegralT (whose pops
+// never need a region's value before the round's last one, so the cuts come after them, together).
+// What bounds it: the chain of heap steps and rounds of an integral (~1.3 ms alone), hidden by the other integrals of the
+// CU, of which there should be many: 16 waves per CU by registers, so BLOCK = 128 (8 integrals) when there are integrals
+// to fill them, 256 (4) when there are not and an integral's own time counts.  512 cosmologies x 10 radii at 1e-5, 5.4e6
+// regions: 29-41 ms in rounds with the heaps on the host, 10.0 with BLOCK 256, 7.3 with 128; 80 integrals 2.9-3.4 ms in
+// rounds, 2.0 (256), 2.3 (128).
+template <int BLOCK>
+__global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) k_map2_integrals(
+    const TpCosmoConst *__restrict__ cc, const double *__restrict__ tab, int n_z, double zmax,
+    const TpPowerDesc *__restrict__ desc, int n, double reltol, int max_rounds, TpMap2Region *pool,
+    TpMap2Out *__restrict__ out, int *next)
+{
+#pragma clang fp contract(off)
+    __shared__ double key[kMap2Regions];            // heap: errors,
+    __shared__ unsigned short hid[kMap2Regions];    // and their regions
+    __shared__ unsigned short pop[kMap2Regions / 2];  // regions to cut, in the order they left the heap
+    __shared__ double fv[kMap2Chunk * kGm2Pts];
+    __shared__ double sv[kMap2Chunk], se[kMap2Chunk];
+    __shared__ int s_k, s_np, s_end, s_bad;
+    const int t = threadIdx.x;
+    TpMap2Region *P = pool + (size_t)blockIdx.x * kMap2Regions;
+    for (;;) {
+        if (t == 0) {
+            s_k = atomicAdd(next, 1);
+            s_bad = 0;
+        }
+        __syncthreads();
+        const int k = s_k;
+        if (k >= n) return;
+        const TpPowerDesc D = desc[k];
+        const TpCosmoConst &C = cc[D.icosmo];
+        const double *T = tab + (size_t)D.icosmo * 6 * n_z;
+        if (t == 0) {
+            TpMap2Region R{};  // ell in [1, 10 / theta] (apertureStatistics.cu:112-113), z in [0, z_max]
+            const double hi = 10. / D.par;
+            R.c[0] = 0.5 * (1. + hi);
+            R.hw[0] = 0.5 * (hi - 1.);
+            R.c[1] = 0.5 * (0. + zmax);
+            R.hw[1] = 0.5 * (zmax - 0.);
+            R.vol = 2 * R.hw[0] * (2 * R.hw[1]);
+            P[0] = R;
+            pop[0] = 0;
+        }
+        double sval = 0, serr = 0;
+        int nheap = 0, npool = 1, nold = 1, npend = 1, rounds = 0;
+        long long nreg = 0;
+        __syncthreads();
+        for (;;) {
+            // the round's regions: cut region and its new half in turn
+            auto region = [&](int j) { return j & 1 ? nold + (j >> 1) : (int)pop[j >> 1]; };
+            for (int c0 = 0; c0 < npend; c0 += kMap2Chunk) {
+                const int m = min(kMap2Chunk, npend - c0);
+                for (int i = t; i < m * kGm2Pts; i += BLOCK) {
+                    const int r = i / kGm2Pts, p = i - r * kGm2Pts;
+                    const TpMap2Region &R = P[region(c0 + r)];
+                    fv[i] = tp_map2_point<double>(C, T, n_z, tp_gm_coord(R.c[0], R.hw[0], c_gm2_code[p][0]),
+                                                  tp_gm_coord(R.c[1], R.hw[1], c_gm2_code[p][1]), D.par, D.flags,
+                                                  D.sigma, D.ngal);
+                }
+                __syncthreads();
+                if (t < m) {
+                    TpMap2Region &R = P[region(c0 + t)];
+                    const TpRegion2Out o = gm_rule2(R.vol, fv + t * kGm2Pts);
+                    R.val = o.val;
+                    R.split = o.split;
+                    sv[t] = o.val;
+                    se[t] = o.err;
+                    if (o.flag) s_bad = 1;
+                }
+                __syncthreads();
+                if (t == 0) {  // while the others start on the next chunk's points
+                    for (int q = 0; q < m; ++q) {
+                        const double kq = se[q];
+                        sval += sv[q];
+                        serr += kq;
+                        int ins = nheap++;
+                        while (ins) {
+                            const int par = (ins - 1) / 2;
+                            if (kq <= key[par]) break;
+                            key[ins] = key[par];
+                            hid[ins] = hid[par];
+                            ins = par;
+                        }
+                        key[ins] = kq;
+                        hid[ins] = (unsigned short)region(c0 + q);
+                    }
+                }
+            }
+            nreg += npend;
+            ++rounds;
+            __syncthreads();  // every thread is past its use of pop
+            if (t == 0) {
+                int end = 0, np = 0;
+                const double tol = fabs(sval) * reltol;
+                if (s_bad) {
+                    end = 2;
+                } else if (!(serr > 0 && serr > tol)) {
+                    end = 1;
+                } else if (rounds >= max_rounds) {
+                    end = 2;
+                } else {
+                    do {
+                        if (npool + np == kMap2Regions) {
+                            end = 2;
+                            break;
+                        }
+                        const double top = key[0];
+                        pop[np++] = hid[0];
+                        const int nh = --nheap;
+                        const double km = key[nh];
+                        const unsigned short im = hid[nh];
+                        int i = 0, child;
+                        while ((child = 2 * i + 1) < nh) {
+                            const double kc = key[child], k2 = child + 1 < nh ? key[child + 1] : -1.;
+                            int largest = kc <= km ? i : child;
+                            const double kl = kc <= km ? km : kc;
+                            largest = kl < k2 ? child + 1 : largest;
+                            if (largest == i) break;
+                            key[i] = kl < k2 ? k2 : kc;
+                            hid[i] = hid[largest];
+                            i = largest;
+                        }
+                        if (nh) {
+                            key[i] = km;
+                            hid[i] = im;
+                        }
+                        serr -= top;
+                    } while (serr > 0 && serr > tol && nheap);
+                }
+                s_np = np;
+                s_end = end;
+            }
+            __syncthreads();
+            if (s_end) break;
+            const int np = s_np;
+            for (int c0 = 0; c0 < np; c0 += kMap2Chunk * kGm2Pts) {
+                const int m = min(kMap2Chunk * kGm2Pts, np - c0);
+                for (int j = t; j < m; j += BLOCK) {  // classed_version/hcubature.cpp:206-218
+                    TpMap2Region A = P[pop[c0 + j]];
+                    fv[j] = A.val;
+                    const bool d = A.split != 0;
+                    (d ? A.hw[1] : A.hw[0]) *= 0.5;
+                    A.vol *= 0.5;
+                    TpMap2Region B = A;
+                    B.vol = 2 * B.hw[0] * (2 * B.hw[1]);
+                    const double h = d ? A.hw[1] : A.hw[0];
+                    (d ? A.c[1] : A.c[0]) -= h;
+                    (d ? B.c[1] : B.c[0]) += h;
+                    P[pop[c0 + j]] = A;
+                    P[npool + c0 + j] = B;
+                }
+                __syncthreads();
+                if (t == 0)
+                    for (int q = 0; q < m; ++q) sval -= fv[q];
+                __syncthreads();
+            }
+            nold = npool;
+            npool += np;
+            npend = 2 * np;
+        }
+        if (s_end == 1) {  // the sums anew, in heap order (classed_version/hcubature.cpp:1000-1008)
+            nheap = npool;  // all regions are in the heap
+            double v = 0, e = 0;
+            for (int c0 = 0; c0 < nheap; c0 += kMap2Chunk * kGm2Pts) {
+                const int m = min(kMap2Chunk * kGm2Pts, nheap - c0);
+                __syncthreads();
+                for (int j = t; j < m; j += BLOCK) fv[j] = P[hid[c0 + j]].val;
+                __syncthreads();
+                if (t == 0)
+                    for (int q = 0; q < m; ++q) {
+                        v += fv[q];
+                        e += key[c0 + q];
+                    }
+            }
+            if (t == 0) out[k] = TpMap2Out{v, e, nreg, rounds, 0};
+        } else if (t == 0) {
+            out[k] = TpMap2Out{0., 0., nreg, rounds, 1};
+        }
+        // Without a barrier here the compiler joins this thread 0 branch with the one at the loop's head and sends the
+        // first wave's other lanes round the loop ahead of thread 0.
+        __syncthreads();
+    }
 }
 
 // Pell: one wave per multipole.  Lane j < 48 evaluates the node pair j (z = cx -+ dx x_j); lane 0
@@ -862,6 +1065,8 @@ int regions_batch(tp_ctx *ctx, const std::vector<TpPowerDesc> &desc, const doubl
     return 0;
 }
 
+double map2_post(double v) { return v / 2. / tpd::kPi; }  // apertureStatistics.cu:135
+
 // <Map^2> rounds: one thread per (region, point), then one thread per region for the rule.
 int map2_regions(tp_ctx *ctx, const tp_cosmo *c, const std::vector<TpPowerDesc> &desc, const double *lo,
                  const double *hi, double reltol, double *out, double *err, long long *neval)
@@ -879,8 +1084,113 @@ int map2_regions(tp_ctx *ctx, const tp_cosmo *c, const std::vector<TpPowerDesc> 
         return 0;
     };
     return regions_batch<2>(ctx, desc, lo, hi, reltol, kGm2Pts, launch,
-                            [](double v) { return v / 2. / tpd::kPi; },  // apertureStatistics.cu:135
-                            "<Map^2> integrand", out, err, neval);
+                            map2_post, "<Map^2> integrand", out, err, neval);
+}
+
+// <Map^2> integrals: whole on the device, in launches of at most kMap2Slice; the few it cannot finish there (see
+// TpMap2Out::host) from their start by the rounds above, whose limits and errors they then meet.  Below kMap2Few
+// integrals the chip is empty either way and the host's heaps are faster than thread 0's (1 integral 0.9 ms in rounds,
+// 1.4 on the device; 8: 1.4-1.75 and 1.6; 16: 2.0 and 1.65).  Below kMap2Reltol integrals outgrow kMap2Regions (held at
+// most: 690 regions at 1e-5, 1250 at 3e-6, 2030 at 1e-6), so that their work there is lost (40 integrals, 1e-7: 5-6 ms in
+// rounds, 12 with the device first).
+constexpr size_t kMap2Few = 16;
+constexpr double kMap2Reltol = 5e-6;
+constexpr int kMap2Slice = 65536;
+int map2_integrals(tp_ctx *ctx, const tp_cosmo *c, const std::vector<TpPowerDesc> &desc, const double *lo,
+                   const double *hi, double reltol, double *out, double *err, long long *neval)
+{
+    using clk = std::chrono::steady_clock;
+    const auto t0 = clk::now();
+    const size_t n = desc.size();
+    if (n < kMap2Few || !(reltol >= kMap2Reltol)) return map2_regions(ctx, c, desc, lo, hi, reltol, out, err, neval);
+    tp_batch_stats st{};
+    int rc, ncu = 0;
+    TP_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, ctx->device));
+    TpLane &L = ctx->lane[0];
+    if ((rc = L.create())) return rc;
+    const size_t slice = std::min(n, (size_t)kMap2Slice);
+    const bool wide = slice <= (size_t)ncu * 4;  // 256 threads, 4 workgroups per CU; else 128 and 8
+    const size_t slots = std::min(slice, (size_t)ncu * (wide ? 4 : 8));
+    if ((rc = ctx->d_desc.ensure(slice * sizeof(TpPowerDesc))) ||
+        (rc = L.d_fvals.ensure(slots * kMap2Regions * sizeof(TpMap2Region))) ||
+        (rc = L.h_rout.ensure(slice * sizeof(TpMap2Out))))
+        return rc;
+    std::vector<TpMap2Out> res(n);
+    std::vector<size_t> rest;
+    auto limit = [&] {
+        return tp_set_error(TP_ECAPACITY, "<Map^2> integrand: region limit reached (integrals not converging)");
+    };
+    for (size_t i0 = 0; i0 < n; i0 += slice) {
+        const size_t m = std::min(slice, n - i0);
+        TP_HIP(hipMemsetAsync(ctx->d_flag.p, 0, sizeof(int), ctx->stream));
+        TP_HIP(hipMemcpyAsync(ctx->d_desc.p, desc.data() + i0, m * sizeof(TpPowerDesc), hipMemcpyHostToDevice,
+                              ctx->stream));
+        TP_HIP(hipEventRecord(ctx->ev0, ctx->stream));
+        hipLaunchKernelGGL(wide ? k_map2_integrals<256> : k_map2_integrals<128>, dim3((unsigned)std::min(m, slots)),
+                           dim3(wide ? 256 : 128), 0, ctx->stream,
+                           c->d_const, c->d_tab, c->n_z, c->z_max, (const TpPowerDesc *)ctx->d_desc.p, (int)m, reltol,
+                           (int)std::min(ctx->max_rounds, 0x7fffffffLL), (TpMap2Region *)L.d_fvals.p,
+                           (TpMap2Out *)L.h_rout.dp, (int *)ctx->d_flag.p);
+        TP_HIP(hipGetLastError());
+        TP_HIP(hipEventRecord(ctx->ev1, ctx->stream));
+        const auto tw = clk::now();
+        TP_HIP(hipStreamSynchronize(ctx->stream));
+        st.wait_ms += std::chrono::duration<double, std::milli>(clk::now() - tw).count();
+        float ms = 0;
+        TP_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
+        st.kernel_ms += ms;
+        st.launches += 1;
+        const TpMap2Out *h = (const TpMap2Out *)L.h_rout.p;
+        for (size_t i = 0; i < m; ++i) {
+            res[i0 + i] = h[i];
+            if (h[i].host) rest.push_back(i0 + i);
+            st.regions += h[i].nreg;
+            st.rounds = std::max(st.rounds, (long long)h[i].rounds);
+        }
+        if (st.regions > ctx->max_regions) return limit();
+    }
+    st.integrand_ms = st.integrand_sum_ms = st.kernel_ms;
+    st.points = st.regions * kGm2Pts;
+    if (!rest.empty()) {
+        const size_t nr = rest.size();
+        std::vector<TpPowerDesc> rd(nr);
+        std::vector<double> rlo(2 * nr), rhi(2 * nr), rv(nr), re(nr);
+        std::vector<long long> rn(nr);
+        for (size_t i = 0; i < nr; ++i) {
+            rd[i] = desc[rest[i]];
+            for (int d = 0; d < 2; ++d) {
+                rlo[2 * i + d] = lo[2 * rest[i] + d];
+                rhi[2 * i + d] = hi[2 * rest[i] + d];
+            }
+            st.regions -= res[rest[i]].nreg;
+        }
+        if ((rc = map2_regions(ctx, c, rd, rlo.data(), rhi.data(), reltol, rv.data(), re.data(), rn.data()))) return rc;
+        for (size_t i = 0; i < nr; ++i) {
+            out[rest[i]] = rv[i];
+            if (err) err[rest[i]] = re[i];
+            if (neval) neval[rest[i]] = rn[i];
+        }
+        const tp_batch_stats &r = ctx->stats;
+        st.rounds = std::max(st.rounds, r.rounds);
+        st.launches += r.launches;
+        st.regions += r.regions;
+        st.points = st.regions * kGm2Pts;
+        st.kernel_ms += r.kernel_ms;
+        st.integrand_ms += r.integrand_ms;
+        st.integrand_sum_ms += r.integrand_sum_ms;
+        st.host_ms += r.host_ms;
+        st.wait_ms += r.wait_ms;
+        if (st.regions > ctx->max_regions) return limit();
+    }
+    for (size_t i = 0; i < n; ++i) {
+        if (res[i].host) continue;
+        out[i] = map2_post(res[i].val);
+        if (err) err[i] = map2_post(res[i].err);
+        if (neval) neval[i] = res[i].nreg * kGm2Pts;
+    }
+    st.wall_ms = std::chrono::duration<double, std::milli>(clk::now() - t0).count();
+    ctx->stats = st;
+    return 0;
 }
 
 // T1 rounds: one launch of k_t1_regions (points, cached Pell and rule in one kernel).
@@ -1012,7 +1322,7 @@ extern "C" int tp_map2_batch(tp_ctx *ctx, const tp_cosmo *c, size_t n, const int
         lo[2 * i + 1] = 0;             // z range [0, z_max]
         hi[2 * i + 1] = c->z_max;
     }
-    return map2_regions(ctx, c, desc, lo.data(), hi.data(), reltol, out, err, neval);
+    return map2_integrals(ctx, c, desc, lo.data(), hi.data(), reltol, out, err, neval);
 }
 
 int tp_build_pnodes(tp_ctx *ctx, tp_cosmo *c)
