@@ -1,19 +1,20 @@
 // tp_map3.hip -- gfx950 kernels of the <Map^3> integrand path.
 //
-//  * bispec_q<T>: BiHalofit (Takahashi et al. 2020, eqs. B4-B9) at one Limber
+//  * the node (tp_device.h): BiHalofit (Takahashi et al. 2020, eqs. B4-B9) at one Limber
 //    z-node, restating classed_version/bispectrum.cpp:166-236 (with F2 :614-633
 //    and the Eisenstein & Hu P(k) :811-841) in terms of the dimensionless
 //    wavenumbers q = k r_sigma.  Everything that depends on z only comes from a
 //    per-node record (TpNodeT) that the table builder evaluated once in FP64.
-//  * bkappa_sum<T>: the 96-node Limber sum of classed_version/bispectrum.cpp:
-//    238-286 / 1010-1020, accumulated in FP64.  T = double is the plain path;
+//  * the 96-node Limber sum of classed_version/bispectrum.cpp: 238-286 /
+//    1010-1020, accumulated in FP64.  T = double is the plain path;
 //    T = float runs the bispectrum in FP32 (native v_exp_f32 / v_log_f32).
-//    Node records are wave-uniform, so they are read through scalar loads.
-//  * map3 point kernel: classed_version/apertureStatistics.cpp:16-28.
+//  * point kernels (k_points, k_points_nodes): rows of B_kappa or of the <Map^3>
+//    integrand, classed_version/apertureStatistics.cpp:16-28.
 //  * region kernels: Genz-Malik degree-7/5 rule (classed_version/hcubature.cpp:
-//    456-577) for many 3-D regions of many integrals per launch -- one thread
-//    per (region, point), then one thread per region for the rule sums, in the
-//    reference's summation order.
+//    456-577) for many 3-D regions of many integrals per launch -- the points
+//    (a thread or several waves per point, or P_E terms shared by a region's
+//    points), then one thread per region for the rule sums, in the reference's
+//    summation order.
 #include <cmath>
 #include <vector>
 

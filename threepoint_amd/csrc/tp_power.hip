@@ -13,11 +13,12 @@
 // unfinished integrals and one launch evaluates all their rule points (15 Gauss-Kronrod points in 1-D,
 // 17 / 33 / 57 Genz-Malik points in 2-D / 3-D / 4-D); each integral's heap advances with the decision
 // sequence of the reference's one-at-a-time hcubature.  P_kappa and the 4-D covariance apply the rules
-// on the host; <Map^2> and T1 apply them on the device (bit-identical arithmetic order).
+// on the host; <Map^2> and T1 apply them on the device (bit-identical arithmetic order), and a batch of <Map^2>
+// integrals runs on the device altogether, heaps included (k_map2_integrals).
 //
 // Per point the integrand is one table interpolation, the Halofit z-coefficients (pow), the k-part in
 // log space and the filter: transcendental-bound FP64 work on a few doubles of input, so a launch is
-// bounded by its FP64 issue rate, and the rounds by the host.
+// bounded by its FP64 issue rate, and rounds of cheap points by the host.
 #include <algorithm>
 #include <chrono>
 #include <cmath>
