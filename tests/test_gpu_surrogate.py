@@ -250,7 +250,23 @@ def test_surrogate_form_within_1e3_of_fp64(gpu_ctx, fid_nz, workload):
 
 @pytest.mark.parametrize("M", [192, 4160])
 def test_mlp_gradients_of_ragged_batches(gpu_ctx, M):
-    """Batches whose weight-gradient splits end inside a 64-row stage (192 rows: splits of 192; 4160: 16 splits of 288
-    rows and a last one that is shorter) and whose column sums have a partial last pass, against the oracle at the
+    """Batches whose column sums have a partial last pass, the larger one with weight-gradient splits that end inside a
+    64-row stage (192 rows: one split; 4160: 14 splits of 288 rows and one of 128), against the oracle at the
     tolerance of test_mlp_gradients_match_cpu_oracle."""
     test_mlp_gradients_match_cpu_oracle(gpu_ctx, M)
+
+
+@pytest.mark.parametrize("first, M", [(9472, 1216), (4096, 192), (16128, 15872)])
+def test_mlp_gradients_do_not_depend_on_earlier_batches(first, M):
+    """A context keeps the workspace of its largest batch.  A smaller batch after it is split by its own size alone, so
+    it stays inside that workspace (37, 16 and 63 splits' worth) and has the bits it has in a fresh context."""
+    rng = np.random.default_rng(M)
+    p = rng.normal(0, 0.08, MO.NPARAM)
+    X, T = rng.uniform(-1, 1, (first, MO.NIN)), rng.normal(0, 1, first)
+    used, fresh = tp.Context(), tp.Context()
+    _gpu_loss_grad(used, p, X, T)
+    l1, g1 = _gpu_loss_grad(used, p, X[:M], T[:M])
+    l0, g0 = _gpu_loss_grad(fresh, p, X[:M], T[:M])
+    assert np.array_equal(g1, g0) and abs(l1 / l0 - 1) < 1e-12
+    used.close()
+    fresh.close()

@@ -36,6 +36,7 @@
 #include <vector>
 
 #include "tp_device.h"
+#include "tp_mlp_split.h"
 
 namespace {
 
@@ -528,7 +529,6 @@ struct TpSurrogate {
     unsigned short *A[4] = {nullptr, nullptr, nullptr, nullptr};
     unsigned short *dZ[4] = {nullptr, nullptr, nullptr, nullptr};
     float *parts = nullptr;
-    int nsplit = 0;
     double *d_loss = nullptr;
     SurBox box{};
     float t_mean = 0, t_std = 1;
@@ -568,8 +568,7 @@ static int sur_ensure_batch(TpSurrogate *s, int rows)
         TP_HIP(hipMalloc(&s->A[i], (size_t)cap * H * sizeof(unsigned short)));
         TP_HIP(hipMalloc(&s->dZ[i], (size_t)cap * H * sizeof(unsigned short)));
     }
-    s->nsplit = std::max(1, std::min(64, cap / 256));
-    TP_HIP(hipMalloc(&s->parts, (size_t)3 * s->nsplit * H * H * sizeof(float)));
+    TP_HIP(hipMalloc(&s->parts, (size_t)3 * tp_wgrad_max_splits(cap) * H * H * sizeof(float)));
     s->cap = cap;
     return 0;
 }
@@ -615,10 +614,7 @@ static int sur_backward(hipStream_t st, TpSurrogate *s, int M)
         hipLaunchKernelGGL(k_gemm_rows<true>, dim3(M / GM, H / GN), dim3(256), 0, st, s->dZ[l + 1],
                            s->Wb + (size_t)(NLAYER_MFMA + l) * H * H, (const float *)nullptr, s->Z[l], s->dZ[l]);
     // then every gradient: the weights' (split over the batch) and the sums
-    constexpr int kc0 = 32;  // splits are whole multiples of this many rows
-    int ns = std::max(1, std::min(s->nsplit, M / kc0));
-    const int kc = ((M / ns + kc0 - 1) / kc0) * kc0;
-    ns = (M + kc - 1) / kc;
+    const TpWgradSplit sp = tp_wgrad_split(M);  // sp.n <= tp_wgrad_max_splits(s->cap)
     WgradArgs wa{};
     SmallGradArgs sa{};
     for (int l = 0; l < 3; ++l) {
@@ -629,9 +625,9 @@ static int sur_backward(hipStream_t st, TpSurrogate *s, int M)
     sa.A4 = s->A[3];
     sa.X = s->X;
     sa.dy = s->dy;
-    hipLaunchKernelGGL(k_gemm_wgrad, dim3(H / 64, H / 64, 3 * ns), dim3(256), 0, st, wa, M, kc, ns, s->parts);
+    hipLaunchKernelGGL(k_gemm_wgrad, dim3(H / 64, H / 64, 3 * sp.n), dim3(256), 0, st, wa, M, sp.rows, sp.n, s->parts);
     hipLaunchKernelGGL(k_small_grads, dim3(kSumBlocks, 6), dim3(256), 0, st, sa, M, s->G);
-    hipLaunchKernelGGL(k_reduce_parts, dim3(H * H / 256, 3), dim3(256), 0, st, s->parts, ns, s->G);
+    hipLaunchKernelGGL(k_reduce_parts, dim3(H * H / 256, 3), dim3(256), 0, st, s->parts, sp.n, s->G);
     TP_HIP(hipGetLastError());
     return 0;
 }
