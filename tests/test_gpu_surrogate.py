@@ -270,3 +270,24 @@ def test_mlp_gradients_do_not_depend_on_earlier_batches(first, M):
     assert np.array_equal(g1, g0) and abs(l1 / l0 - 1) < 1e-12
     used.close()
     fresh.close()
+
+
+def test_mlp_batch_that_does_not_fit_leaves_the_context_usable():
+    """A batch whose workspace cannot be allocated (2^31 - 64 rows: 2 TiB a layer; the rows are not read before) or
+    whose row count no kernel index holds is refused, and the next batch computes what it computes in a fresh
+    context."""
+    rng = np.random.default_rng(5)
+    p = rng.normal(0, 0.08, MO.NPARAM)
+    X, T = rng.uniform(-1, 1, (256, MO.NIN)), rng.normal(0, 1, 256)
+    ctx, fresh = tp.Context(), tp.Context()
+    _gpu_loss_grad(ctx, p, X, T)
+    few, g, loss = np.zeros((64, MO.NIN), np.float32), np.zeros(MO.NPARAM, np.float32), ctypes.c_double()
+    for n in (2 ** 31 - 64, 2 ** 31, 2 ** 32 + 64):
+        rc = tp.lib().tp_mlp_loss_grad(ctx.h, n, few.ctypes.data_as(_fp), few.ctypes.data_as(_fp), ctypes.byref(loss),
+                                       g.ctypes.data_as(_fp))
+        assert rc != 0, n
+    l1, g1 = _gpu_loss_grad(ctx, p, X, T)
+    l0, g0 = _gpu_loss_grad(fresh, p, X, T)
+    assert np.array_equal(g1, g0) and abs(l1 / l0 - 1) < 1e-12
+    ctx.close()
+    fresh.close()

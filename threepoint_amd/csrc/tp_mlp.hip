@@ -552,23 +552,38 @@ static int sur_alloc(TpSurrogate *s)
     return 0;
 }
 
-static int sur_ensure_batch(TpSurrogate *s, int rows)
+// Room for `rows` rows.  Where an allocation fails, what had been freed is not left behind as a pointer or a capacity:
+// the next call, whatever its size, allocates anew, and what had been allocated for this one is given back.
+static int sur_ensure_batch(TpSurrogate *s, size_t rows)
 {
-    if (rows <= s->cap) return 0;
-    int cap = ((rows + 63) / 64) * 64;
-    auto F = [](void *p) { if (p) (void)hipFree(p); };
-    F(s->X); F(s->T); F(s->Y); F(s->dy); F(s->parts);
-    for (int i = 0; i < 4; ++i) { F(s->Z[i]); F(s->A[i]); F(s->dZ[i]); }
-    TP_HIP(hipMalloc(&s->X, (size_t)cap * NIN * sizeof(float)));
-    TP_HIP(hipMalloc(&s->T, (size_t)cap * sizeof(float)));
-    TP_HIP(hipMalloc(&s->Y, (size_t)cap * sizeof(float)));
-    TP_HIP(hipMalloc(&s->dy, (size_t)cap * sizeof(float)));
-    for (int i = 0; i < 4; ++i) {
-        TP_HIP(hipMalloc(&s->Z[i], (size_t)cap * H * sizeof(float)));
-        TP_HIP(hipMalloc(&s->A[i], (size_t)cap * H * sizeof(unsigned short)));
-        TP_HIP(hipMalloc(&s->dZ[i], (size_t)cap * H * sizeof(unsigned short)));
+    if (rows <= (size_t)s->cap) return 0;
+    if (rows > 0x7fffffc0u) return tp_set_error(TP_ECAPACITY, "training batch: more than 2^31 - 64 rows");
+    const int cap = (int)((rows + 63) / 64 * 64);
+    hipError_t e = hipSuccess;
+    auto renew = [&](auto *&p, size_t n) {
+        if (p) (void)hipFree(p);
+        p = nullptr;
+        if (e == hipSuccess) e = hipMalloc(&p, n * sizeof(*p));
+    };
+    auto renew_all = [&] {
+        renew(s->X, (size_t)cap * NIN);
+        renew(s->T, (size_t)cap);
+        renew(s->Y, (size_t)cap);
+        renew(s->dy, (size_t)cap);
+        for (int i = 0; i < 4; ++i) {
+            renew(s->Z[i], (size_t)cap * H);
+            renew(s->A[i], (size_t)cap * H);
+            renew(s->dZ[i], (size_t)cap * H);
+        }
+        renew(s->parts, (size_t)3 * tp_wgrad_max_splits(cap) * H * H);
+    };
+    s->cap = 0;
+    renew_all();
+    if (e != hipSuccess) {
+        renew_all();  // frees only
+        (void)hipGetLastError();  // reported here, not by the next launch's check
+        return tp_set_error(TP_EHIP, std::string("training batch: hipMalloc: ") + hipGetErrorString(e));
     }
-    TP_HIP(hipMalloc(&s->parts, (size_t)3 * tp_wgrad_max_splits(cap) * H * H * sizeof(float)));
     s->cap = cap;
     return 0;
 }
@@ -720,7 +735,7 @@ extern "C" int tp_mlp_loss_grad(tp_ctx *ctx, size_t n, const float *x, const flo
     if (!ctx->sur) return tp_set_error(TP_EINVAL, "tp_mlp_loss_grad: set parameters first");
     TP_HIP(hipSetDevice(ctx->device));
     TpSurrogate *s = ctx->sur;
-    int rc = sur_ensure_batch(s, (int)n);
+    int rc = sur_ensure_batch(s, n);
     if (rc) return rc;
     hipStream_t st = ctx->stream;
     TP_HIP(hipMemcpyAsync(s->X, x, n * NIN * sizeof(float), hipMemcpyHostToDevice, st));
@@ -1278,7 +1293,7 @@ extern "C" int tp_surrogate_train(tp_ctx *ctx, const tp_train_config *cfg, tp_tr
     TRY(hipMemcpyAsync(s->P, p0.data(), NPARAM * sizeof(float), hipMemcpyHostToDevice, st));
     TRY(hipMemsetAsync(s->Am, 0, NPARAM * sizeof(float), st));
     TRY(hipMemsetAsync(s->Av, 0, NPARAM * sizeof(float), st));
-    if ((rc = sur_refresh_bf16(st, s)) || (rc = sur_ensure_batch(s, cfg->batch))) {
+    if ((rc = sur_refresh_bf16(st, s)) || (rc = sur_ensure_batch(s, (size_t)cfg->batch))) {
         cleanup();
         return rc;
     }
