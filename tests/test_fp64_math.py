@@ -24,7 +24,10 @@ extern "C" void run(int what, int n, const double *x, double *y, long double *re
         else if (what == 1) { y[i] = tp_fp64_log(x[i]); if (ref) ref[i] = logl(x[i]); }
         else if (what == 2) { y[i] = tp_fp64_rcp(x[i]); if (ref) ref[i] = 1.0L / x[i]; }
         else if (what == 3) { y[i] = tp_fp64_log1p(x[i]); if (ref) ref[i] = log1pl(x[i]); }
-        else { y[i] = tp_fp64_exp10(x[i]); if (ref) ref[i] = powl(10.0L, x[i]); }
+        else if (what == 4) { y[i] = tp_fp64_exp10(x[i]); if (ref) ref[i] = powl(10.0L, x[i]); }
+        else if (what == 5) { y[i] = tp_fp64_exp_any(x[i]); if (ref) ref[i] = expl(x[i]); }
+        else if (what == 6) { y[i] = tp_fp64_exp_low(x[i]); if (ref) ref[i] = expl(x[i]); }
+        else { y[i] = tp_fp64_rcp_any(x[i]); if (ref) ref[i] = 1.0L / x[i]; }
     }
 }
 """
@@ -88,3 +91,21 @@ def test_ends_of_the_range(fp64):
     assert np.all(np.isinf(y[:2])) and np.all(y[2:4] == 0) and y[4] == 1 and np.isnan(y[5])
     y, _ = fp64(1, [1.0])
     assert abs(y[0]) < 2.0 ** -60
+
+
+def test_the_whole_stated_domain_and_the_forms_for_any_argument(fp64):
+    """exp up to 2^30 either way; exp_any and exp_low beyond it, infinities included, and rcp_any at the infinities,
+    each with the bits of the plain form inside its range."""
+    far = np.array([1e4, 1.4e9 / 2, 2.0 ** 30])
+    y, _ = fp64(0, np.concatenate([far, -far]))
+    assert np.all(np.isposinf(y[:3])) and np.all(y[3:] == 0)
+    farther = np.array([1.4e9, 1.5e9, 2.0 ** 31 - 1, 2.1e9, 1e10, 1e15, 1e18, 1e100, 1e300, np.inf])
+    assert np.all(np.isposinf(fp64(5, farther)[0])) and np.all(fp64(5, -farther)[0] == 0)
+    assert np.all(fp64(6, -farther)[0] == 0)
+    y, _ = fp64(7, [np.inf, -np.inf, np.nan])
+    assert y[0] == 0 and not np.signbit(y[0]) and y[1] == 0 and np.signbit(y[1]) and np.isnan(y[2])
+    x = np.random.default_rng(3).uniform(-700, 700, 20000)
+    for form, plain in ((5, 0), (6, 0), (7, 2)):
+        assert np.array_equal(fp64(form, x)[0], fp64(plain, x)[0])
+    e = np.exp(np.random.default_rng(4).uniform(-700, 700, 20000))
+    assert np.array_equal(fp64(7, e)[0], fp64(2, e)[0])

@@ -35,8 +35,16 @@ __device__ __forceinline__ float tp_logf_normal(float x)
 // library's functions, one MI355X: 17 920 <Map^3> integrals 6.98 -> 4.71 s with the series logarithm, 10^6 B_kappa points 6.3 -> 4.8 ms,
 // 8 192 Gamma points of 14 997 terms 4.82 -> 3.04 ms; with the table logarithm 24 x 35 integrals 201 -> 191 ms, the Gamma
 // points 2.81 ms; every integral keeps its point count.  FP32: 24 x 35 integrals 80.5 -> 77.2 ms.
-template <class T> struct TpNodeMath : TpMath<T> {};
-template <> struct TpNodeMath<float> : TpMath<float> {
+// ex_any, ex_low and rcp_any are for the few arguments that can leave the range of the short forms (tp_pse_node,
+// tp_bispec_joint_s): there a node is to stay finite where the library's functions leave it finite, and only there.  They
+// cost 15 of a node's ~490 issues: the Gamma points 2.81 -> 2.87 ms, 36 x 35 integrals 289 -> 292 ms.
+template <class T> struct TpMathAny : TpMath<T> {
+    static __host__ __device__ __forceinline__ T ex_any(T x) { return TpMath<T>::ex(x); }
+    static __host__ __device__ __forceinline__ T ex_low(T x) { return TpMath<T>::ex(x); }
+    static __host__ __device__ __forceinline__ T rcp_any(T x) { return TpMath<T>::rcp(x); }
+};
+template <class T> struct TpNodeMath : TpMathAny<T> {};
+template <> struct TpNodeMath<float> : TpMathAny<float> {
     // __logf without its branches for denormals and infinities (12 instructions to 5, same bits for x >= FLT_MIN):
     // ln 2 times v_log_f32, the product's rounding and the constant's second word added back
     static __device__ __forceinline__ float lg(float x) { return tp_logf_normal(x); }
@@ -45,6 +53,9 @@ template <> struct TpNodeMath<double> {
     static __host__ __device__ __forceinline__ double ex(double x) { return tp_fp64_exp(x); }
     static __host__ __device__ __forceinline__ double lg(double x) { return tp_fp64_log(x); }
     static __host__ __device__ __forceinline__ double rcp(double x) { return tp_fp64_rcp(x); }
+    static __host__ __device__ __forceinline__ double ex_any(double x) { return tp_fp64_exp_any(x); }
+    static __host__ __device__ __forceinline__ double ex_low(double x) { return tp_fp64_exp_low(x); }
+    static __host__ __device__ __forceinline__ double rcp_any(double x) { return tp_fp64_rcp_any(x); }
 };
 
 template <class T>
@@ -177,8 +188,11 @@ __host__ __device__ __forceinline__ T tp_pse_node(const TpNodeT<T> &N, const TpE
     T pq3 = pq * pq * pq;
     T A = T(1) + N.fn * qi * qi;
     T B = T(1) + N.gn * qi + N.hn * qi * qi;
-    T C = (N.mn * M::ex(N.mun * lqi) + N.nn * M::ex(N.nun * lqi)) * (pq3 + T(1));
-    return (A * N.D1sq * pl * C + B * pq3) * M::rcp(B * C);  // eq. B6
+    // mu_n and nu_n are powers of ten of polynomials in n_eff: from n_eff = -0.55 and 2.6 on their products with ln q leave
+    // the range of the short exp, and from n_eff = -1 on B C can overflow at an ordinary ell (the term is then 0).  nu_n ln q
+    // needs its low end only: where it leaves the range above, mu_n ln q is far above it, and C infinite without it.
+    T C = (N.mn * M::ex_any(N.mun * lqi) + N.nn * M::ex_low(N.nun * lqi)) * (pq3 + T(1));
+    return (A * N.D1sq * pl * C + B * pq3) * M::rcp_any(B * C);  // eq. B6
 }
 
 // The parts of the one-halo term that depend on the node and the triangle shape only (eq. B7:
@@ -209,7 +223,7 @@ __host__ __device__ __forceinline__ T tp_bispec_joint_s(const TpNodeT<T> &N, con
         const T qi = q[i], lqi = lq[i];
         T oneh = S.an * M::ex(S.alphan * lqi) + N.bn * M::ex(S.betan * lqi);   // eq. B4
         T cq = N.cn * qi;
-        bs1h *= cq * M::rcp(oneh * (cq + T(1)));
+        bs1h *= cq * M::rcp_any(oneh * (cq + T(1)));  // q^beta_n overflows from q = 1e39 on
         damp *= T(1) + N.en * qi;
     }
     T bs3h = T(2) * ((f2t[0] + N.dn * q[2]) * pse[0] * pse[1] + (f2t[1] + N.dn * q[0]) * pse[1] * pse[2] +

@@ -7,10 +7,12 @@
 //     tp_fp64_exp 14, tp_fp64_log 18, tp_fp64_rcp 6    (here)
 // What is left out is what the node arithmetic never needs: a second word of the logarithm (every one feeds an
 // exponent or a sum whose own rounding is larger), the exactly rounded quotient, and branches for arguments outside the
-// range.  Domain: exp takes any finite argument below 2^31 in magnitude (it overflows to +inf and underflows to 0 there
-// like the library's; a NaN stays a NaN), log any positive normal one (a zero, a denormal, an infinity or a NaN gives
-// some finite number: where one can arrive, another factor of the same value carries it on), rcp any normal number whose
-// reciprocal is normal.  Errors against 80-bit arithmetic: exp 0.91 ulp, exp10 1.19, rcp 0.50, log 0.50 ulp + 2^-60
+// range.  Domain: exp takes any finite argument up to 2^30 in magnitude (it overflows to +inf and underflows to 0 there
+// like the library's; a NaN stays a NaN; beyond 2^31 ln 2 = 1.49e9 the exponent's word wraps), exp10 up to 2^28, log any
+// positive normal one (a zero, a denormal, an infinity or a NaN gives some finite number: where one can arrive, another
+// factor of the same value carries it on), rcp any normal number whose reciprocal is normal.  The forms named _any and
+// _low take what these leave out, for the places it can reach.  Errors against 80-bit arithmetic, in a host build: exp
+// 0.91 ulp, exp10 1.19, rcp 0.50, log 0.50 ulp + 2^-60
 // (tests/test_fp64_math.py).  The logarithm's table is there because its other form, 2 atanh((m - 1) / (m + 1)) with a
 // reciprocal and a degree-15 series, takes 31 instructions to these 15 (25 issues to 18).
 //
@@ -73,15 +75,30 @@ __host__ __device__ __forceinline__ double tp_fp64_exp(double x)
     return tp_fp64_scale(tp_fp64_exp_r(r), t);
 }
 
+// the same for an argument of any size, infinities among them (but a NaN gives a number: a caller has another factor
+// that carries it on), and for one of any size below zero
+__host__ __device__ __forceinline__ double tp_fp64_exp_low(double x) { return tp_fp64_exp(__builtin_fmax(x, -0x1p30)); }
+__host__ __device__ __forceinline__ double tp_fp64_exp_any(double x) { return tp_fp64_exp_low(__builtin_fmin(x, 0x1p30)); }
+
 // hardware reciprocal (2^-27 or better) and one third-order step: error e^3 + the last rounding
-__host__ __device__ __forceinline__ double tp_fp64_rcp(double x)
+__host__ __device__ __forceinline__ double tp_fp64_rcp_seed(double x)
 {
 #ifdef TP_FP64_DEVICE
-    const double r = __builtin_amdgcn_rcp(x);
+    return __builtin_amdgcn_rcp(x);
 #else
-    const double r = (1.0 / x) * (1.0 + 0x1p-27);  // an approximation of no more than the hardware's accuracy
+    return (1.0 / x) * (1.0 + 0x1p-27);  // an approximation of no more than the hardware's accuracy
 #endif
-    const double e = fma(-x, r, 1.0);
+}
+__host__ __device__ __forceinline__ double tp_fp64_rcp(double x)
+{
+    const double r = tp_fp64_rcp_seed(x), e = fma(-x, r, 1.0);
+    return fma(r, fma(e, e, e), r);
+}
+// the same with 1 / +-infinity = +-0: there the seed is 0 and the residual a NaN, which the bound makes -1 and the step
+// then 0; elsewhere the residual is far above -1
+__host__ __device__ __forceinline__ double tp_fp64_rcp_any(double x)
+{
+    const double r = tp_fp64_rcp_seed(x), e = __builtin_fmax(fma(-x, r, 1.0), -1.0);
     return fma(r, fma(e, e, e), r);
 }
 

@@ -455,9 +455,9 @@ __global__ void __launch_bounds__(256) k_gen(const TpNode64 *__restrict__ nodes,
         ok = (l3 >= lmin && l3 <= lmax);
     }
     if (!ok) l1 = l2 = l3 = exp(0.5 * (box.lnl_min + box.lnl_max));
-    // the library's exp and log (TpMath, not the shorter node forms): the samples of a seed stay bit for bit the
+    // the library's exp and log (TpMathAny, not the shorter node forms): the samples of a seed stay bit for bit the
     // ones the shipped network was trained on
-    double b = tp_bkappa_sum<double, TpMath<double>>(nodes + (size_t)ic * TP_NNODES, eh[ic], l1, l2, l3);
+    double b = tp_bkappa_sum<double, TpMathAny<double>>(nodes + (size_t)ic * TP_NNODES, eh[ic], l1, l2, l3);
     const TpCosmoConst &C = cc[ic];
     double cp[5] = {C.om, C.sigma8, C.h, C.w, C.ns};
     make_input(box, l1, l2, l3, cp, X + i * NIN);
