@@ -36,6 +36,17 @@ def test_t1_total_matches_oracle(fid_tables, fid_oracle, flags, lmin):
         assert abs(v[i] / ov - 1) < 1e-10
 
 
+def test_t1_of_far_multipoles(fid_tables, fid_oracle):
+    """Radii so small that the multipoles leave the range of the short FP64 forms take the kernel that branches on it:
+    the oracle's value and point count there, and for the ordinary pair of the same batch the bits it has alone."""
+    far, near = np.full(6, 1e-16), np.array([6, 6, 12, 4, 8, 16], dtype=float) * A
+    v, n = fid_tables.map3_cov_t1(np.array([far, near]), AREA, 0.0, 0.0, NGAL, 0, reltol=1e-3)
+    ov, on = fid_oracle.t1_total(far[:3], far[3:], AREA, 0.0, 0.0, NGAL, 0, 1e-3)
+    assert n[0] == on and abs(v[0] / ov - 1) < 1e-10
+    w, m = fid_tables.map3_cov_t1(near[None, :], AREA, 0.0, 0.0, NGAL, 0, reltol=1e-3)
+    assert m[0] == n[1] and w[0] == v[1]
+
+
 def test_t1_shape_noise_closed_form_on_gpu(fid_tables):
     th = np.array([3.0, 6.0, 12.0]) * A
     pairs = np.repeat(th[:, None], 6, axis=1)

@@ -49,6 +49,27 @@ def test_limber_integrand_matches_oracle(fid_tables, fid_oracle, flags):
     assert r.max() < 1e-12
 
 
+@pytest.mark.parametrize("flags", [0, tp.PK_LINEAR, tp.PK_T17])
+def test_far_wavenumbers_match_oracle(fid_tables, fid_oracle, flags):
+    """k and ell of 1e-60 to 1e60, far outside the range of the short FP64 forms: the values the library's functions
+    give there, to the rounding of (3 + n_s) ln k (550 ulp; the oracle takes powers).  A k that is no number is refused."""
+    rng = np.random.default_rng(13)
+    k = 10 ** rng.uniform(-60, 60, 300)
+    z = rng.uniform(0.05, 3.0, 300)
+    kz = np.stack([k, z], 1)
+    if not flags & tp.PK_T17:
+        name = "linear_pk_at_z" if flags & tp.PK_LINEAR else "pk_nonlinear"
+        o = np.array([fid_oracle.scalar(name, *p) for p in kz])
+        assert rel(fid_tables.pk_at_z(kz, flags=flags), o).max() < 1e-11
+    o = np.array([fid_oracle.scalar("limber_pkappa", *p, flags) for p in kz])
+    assert rel(fid_tables.limber_pkappa(kz, flags=flags), o).max() < 1e-11
+    o = np.array([fid_oracle.scalar("pell", l, 0.0, 1.0, flags) for l in k])
+    assert rel(fid_tables.pell(k, flags=flags), o).max() < 1e-11
+    for call in (fid_tables.pk_at_z, fid_tables.limber_pkappa):
+        with pytest.raises(tp.TpError, match="non-finite"):
+            call(np.array([[-1.0, 1.0]]), flags=flags)
+
+
 @pytest.mark.parametrize("flags,sigma", [(0, 0.0), (tp.PK_T17, 0.0), (0, 0.3)])
 def test_pell_matches_oracle(fid_tables, fid_oracle, flags, sigma):
     """sigma = 0.3 with the reference's default density n (bispectrum.hpp:120-121, integer division

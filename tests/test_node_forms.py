@@ -1,7 +1,7 @@
-"""The short FP64 forms of the z-node arithmetic against the C library's, both from the kernels' own functions
-(tp_bispec_node of threepoint_amd/csrc/tp_device.h) built for the host: over every size of ell and every n_eff, far
-outside a survey's too, the short forms give a number where the library's give one, to rounding, and none where those
-give none (a call with a non-finite value is refused)."""
+"""The short FP64 forms of the bispectrum and power-spectrum arithmetic against the C library's, both from the kernels'
+own functions (threepoint_amd/csrc/tp_device.h, tp_power_dev.h) built for the host: over every size of ell and every
+n_eff, far outside a survey's too, the short forms give a number where the library's give one, to rounding, and none
+where those give none (a call with a non-finite value is refused)."""
 import ctypes
 import os
 import subprocess
@@ -12,7 +12,7 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 SRC = r"""
-#include "tp_device.h"
+#include "tp_power_dev.h"
 // the z-only factors of BiHalofit (Takahashi et al. 2020, app. B)
 static TpNode64 node(double D1, double sigma8, double rs, double ne, double fK, double h, double ns, double norm)
 {
@@ -49,6 +49,54 @@ extern "C" void run(int n, const double *a, int nk, const double *k, const doubl
         for (int j = 0; j < 3; ++j) { q[j] = P.l[j] * N.ks; lq[j] = P.ll[j] + N.lnks; }
         lib[i] = N.wz * tp_bispec_node<double, TpMathAny<double>>(N, E, q, lq, P.f2t, P.lr1, P.r2);
         fast[i] = N.wz * tp_bispec_node<double>(N, E, q, lq, P.f2t, P.lr1, P.r2);
+    }
+}
+
+// a double whose functions are the library's: the power-spectrum templates take the short forms for double only
+struct Lib {
+    double v;
+    Lib(double x = 0) : v(x) {}
+};
+static Lib operator+(Lib a, Lib b) { return a.v + b.v; }
+static Lib operator-(Lib a, Lib b) { return a.v - b.v; }
+static Lib operator*(Lib a, Lib b) { return a.v * b.v; }
+static Lib operator/(Lib a, Lib b) { return a.v / b.v; }
+static Lib operator-(Lib a) { return -a.v; }
+static Lib pow(Lib a, Lib b) { return std::pow(a.v, b.v); }
+static Lib exp(Lib a) { return std::exp(a.v); }
+static Lib log(Lib a) { return std::log(a.v); }
+static Lib sqrt(Lib a) { return std::sqrt(a.v); }
+static Lib log1p(Lib a) { return std::log1p(a.v); }
+static Lib fabs(Lib a) { return std::fabs(a.v); }
+static double tp_dbl(Lib a) { return a.v; }
+
+// rows of h, n_s, norm, Omega_m, w, ell (or k), z; form 0: the Limber integrand, 1: P(k, z), 2: the precomputed z-node,
+// 3: the same without its branch for a far k
+extern "C" void power(int n, const double *a, const double *tab, int n_z, int flags, int form, double *lib, double *fast)
+{
+    for (int i = 0; i < n; ++i, a += 7) {
+        TpCosmoConst C{};
+        C.h = a[0]; C.ns = a[1]; C.norm = a[2]; C.om = a[3]; C.ow = 1 - a[3]; C.w = a[4]; C.zmax = 3; C.n_z = n_z;
+        C.eh_sqrt_alnu = 0.9; C.eh_sh = 110; C.eh_omh2 = a[3] * a[0] * a[0]; C.eh_theta2 = 1.02; C.eh_cL = 2;
+        C.limber_pref = 1e-9;
+        if (form == 1) {
+            TpZAtT<Lib> Z;
+            TpZAtT<double> Y;
+            tp_z_at<Lib>(tab, n_z, 3, a[6], &Z);
+            tp_z_at<double>(tab, n_z, 3, a[6], &Y);
+            lib[i] = tp_pk_at<Lib>(C, Z, a[5], a[6], flags).v;
+            fast[i] = tp_pk_at<double>(C, Y, a[5], a[6], flags);
+            continue;
+        }
+        lib[i] = tp_limber_pk<Lib>(C, tab, n_z, a[5], a[6], flags).v;
+        if (form == 0) {
+            fast[i] = tp_limber_pk<double>(C, tab, n_z, a[5], a[6], flags);
+            continue;
+        }
+        TpPNode N;
+        tp_pnode_make(C, tab, n_z, a[6], &N);
+        fast[i] = form == 2 ? tp_limber_pk_node<true>(C, N, a[5], log(a[5]), flags)
+                            : tp_limber_pk_node<false>(C, N, a[5], log(a[5]), flags);
     }
 }
 """
@@ -96,3 +144,34 @@ def test_short_forms_are_finite_where_the_library_forms_are(forms, ne, ell, tabu
     d = np.abs(fast[seen] / lib[seen] - 1)
     print("finite %.3f, largest difference %.1e" % (fin.mean(), d.max()))
     assert d.max() < 1e-11
+
+
+@pytest.fixture(scope="module")
+def z_tables():
+    from _oracle import Oracle
+    from threepoint_amd import workloads as W
+    t = Oracle(W.fiducial(), W.fiducial_nz()).tables()
+    return np.concatenate([t[k] for k in ("f_K", "g", "D1", "r_sigma", "n_eff", "ncur")]), len(t["f_K"])
+
+
+# The tolerance: as above, with one power (1 + Delta^2)^beta, beta < 5, over another.  Form 3 is for the multipoles of T1,
+# up to 1e15 and down to where a bisected domain could reach.
+@pytest.mark.parametrize("form, ell", [(0, (-1, 6)), (0, (-300, 300)), (1, (-6, 3)), (1, (-300, 300)), (2, (-1, 6)),
+                                       (2, (-300, 300)), (3, (-65, 15))])
+@pytest.mark.parametrize("flags", [0, 1, 2, 3])
+def test_power_spectrum_of_any_wavenumber(forms, z_tables, form, ell, flags):
+    n, rng = 100000, np.random.default_rng(2)
+    a = np.column_stack([rng.uniform(0.5, 0.9, n), rng.uniform(0.8, 1.2, n), 10 ** rng.uniform(-5, -3, n),
+                         rng.uniform(0.1, 0.9, n), rng.uniform(-1.5, -0.5, n), 10 ** rng.uniform(*ell, n),
+                         rng.uniform(0.02, 3, n)])
+    tab, n_z = z_tables
+    lib, fast = np.empty(n), np.empty(n)
+    a_, t_, l_, f_ = (v.ctypes.data_as(ctypes.c_void_p) for v in (a, tab, lib, fast))
+    forms.power(n, a_, t_, n_z, flags, form, l_, f_)
+    fin = np.isfinite(lib)
+    assert fin.sum() > 1000
+    assert np.array_equal(np.isfinite(fast), fin)
+    seen = fin & (np.abs(lib) > 1e-280)
+    d = np.abs(fast[seen] / lib[seen] - 1)
+    print("finite %.3f, largest difference %.1e" % (fin.mean(), d.max()))
+    assert d.max() < 5e-12

@@ -66,6 +66,7 @@ __device__ __forceinline__ double uhat(double eta)
 
 // Pell from the z-node records N[96] (pairs 2j, 2j+1 at cx -+ dx x_j): the cuda_version's device Pell
 // (bispectrum.cu:511-529), node pairs added in the reference's order (GQ96_of_Pk, bispectrum.cpp:1034-1046).
+template <bool ANY = true>
 __device__ double pell_nodes(const TpCosmoConst &C, const TpPNode *__restrict__ N, double ell, int flags, double dx,
                              double shot)
 {
@@ -74,8 +75,8 @@ __device__ double pell_nodes(const TpCosmoConst &C, const TpPNode *__restrict__ 
     const double lell = log(ell);
     double q = 0;
     for (int j = 0; j < 48; ++j)
-        q += c_pgl_w[j] * (tp_limber_pk_node(C, N[2 * j], ell, lell, flags) +
-                           tp_limber_pk_node(C, N[2 * j + 1], ell, lell, flags));
+        q += c_pgl_w[j] * (tp_limber_pk_node<ANY>(C, N[2 * j], ell, lell, flags) +
+                           tp_limber_pk_node<ANY>(C, N[2 * j + 1], ell, lell, flags));
     return q * dx + shot;
 }
 
@@ -266,7 +267,11 @@ template <bool F32> struct T1Shape {
 };
 constexpr int kT1Pell = 14 + TP_NPTS_GM3;     // Pell per region
 
-template <bool F32>  // F32: the Pell from the FP32 node records (pell_nodes32)
+// F32: the Pell from the FP32 node records (pell_nodes32); ANY: pell_nodes for multipoles of any size.  The rule: without
+// it up to kT1OrdinaryEll, where k = ell / f_K stays below 3e19 h/Mpc (f_K > 0.03 Mpc/h from the first z that counts on)
+// and, ell being a rule point of a bisected [lmin, lmax], above the 1e-70 at which the short forms would underflow.
+constexpr double kT1OrdinaryEll = 1e15;
+template <bool F32, bool ANY>
 __global__ void __launch_bounds__(T1Shape<F32>::block) k_t1_regions(const TpCosmoConst *__restrict__ cc,
                                                     const TpPNode *__restrict__ pnode,
                                                     const TpPNode32 *__restrict__ pnode32, double dx,
@@ -304,7 +309,7 @@ __global__ void __launch_bounds__(T1Shape<F32>::block) k_t1_regions(const TpCosm
                 if (F32)
                     v = pell_nodes32(pnode32 + (size_t)D.icosmo * TP_NNODES, ell, D.flags, dx, shot);
                 else
-                    v = pell_nodes(cc[D.icosmo], pnode + (size_t)D.icosmo * TP_NNODES, ell, D.flags, dx, shot);
+                    v = pell_nodes<ANY>(cc[D.icosmo], pnode + (size_t)D.icosmo * TP_NNODES, ell, D.flags, dx, shot);
             }
         }
         pl[rr][k] = v;
@@ -1198,13 +1203,16 @@ int map2_integrals(tp_ctx *ctx, const tp_cosmo *c, const std::vector<TpPowerDesc
 int t1_regions(tp_ctx *ctx, const tp_cosmo *c, const std::vector<TpPowerDesc> &desc, const double *lo,
                const double *hi, double reltol, double area, int mode, double *out, long long *neval)
 {
+    bool any = false;
+    for (const TpPowerDesc &D : desc) any |= !(D.lmax <= kT1OrdinaryEll);
     auto launch = [&](size_t nreg, const TpRegion *d_reg, TpRegionOut *d_out, double *, hipStream_t st,
                       hipEvent_t evm) -> int {
         const bool f32 = mode == TP_MODE_FP32;
         const int nr = f32 ? T1Shape<true>::reg : T1Shape<false>::reg;
         const size_t nblk = (nreg + nr - 1) / nr;
         if (nblk > 0x7fffffffu) return tp_set_error(TP_ECAPACITY, "T1: too many regions for one launch");
-        hipLaunchKernelGGL(f32 ? k_t1_regions<true> : k_t1_regions<false>, dim3((unsigned)nblk),
+        const auto kern = f32 ? k_t1_regions<true, false> : any ? k_t1_regions<false, true> : k_t1_regions<false, false>;
+        hipLaunchKernelGGL(kern, dim3((unsigned)nblk),
                            dim3(f32 ? T1Shape<true>::block : T1Shape<false>::block), 0, st, c->d_const, (const TpPNode *)c->d_pnode,
                            (const TpPNode32 *)c->d_pnode32, c->z_max / 2, (const TpPowerDesc *)ctx->d_desc.p, d_reg,
                            nreg, d_out);

@@ -115,12 +115,17 @@ __host__ __device__ T tp_pk_eh_log(const TpCosmoConst &C, T k, T lk, double norm
     return C.h * C.h * C.h * pk;
 }
 
+// FP64 takes the short forms of tp_fp64.h, with their quotients merged, for k of 3e-20 to 3e19 h/Mpc: there no power,
+// product or denominator of theirs leaves the range of a double.  Outside (and for a k that is no positive number) it
+// takes the forms below as they stand, with the library's functions, so that any k has the value it has there.
+__host__ __device__ __forceinline__ bool tp_k_ordinary(double lk) { return fabs(lk) < 45.0; }
+
 template <class T>
 __host__ __device__ __forceinline__ T tp_pk_lin_log(const TpCosmoConst &C, T k, T lk)
 {
     if constexpr (std::is_same<T, double>::value) {
         if (C.tab.nk) return tp_pk_table(C.tab, k);
-        return 2 * tpd::kPi * tpd::kPi * tp_delta2_lin(C, 1.0, k, lk) * tp_fp64_rcp(k * k * k);
+        if (tp_k_ordinary(lk)) return 2 * tpd::kPi * tpd::kPi * tp_delta2_lin(C, 1.0, k, lk) * tp_fp64_rcp(k * k * k);
     }
     return tp_pk_eh_log<T>(C, k, lk, C.norm);
 }
@@ -157,16 +162,17 @@ __host__ __device__ __forceinline__ double tp_halofit_k64(const TpCosmoConst &C,
     const double ph = h.a * tp_fp64_exp(h.f1 * 3 * ly) * ysqr * tp_fp64_rcp(den * (ysqr + h.xnu));
     // the damping's argument is the one that leaves the range of the short exp (y up to any ell rs / f_K)
     const double damp = tp_fp64_exp(fmax(-y * 0.25 - ysqr * 0.125, -1000.0));
-    // (a given P(k) may be negative: the library's log1p keeps its NaN below -1)
-    const double l1p = C.tab.nk ? log1p(plin) : tp_fp64_log1p(plin);
-    const double pq = plin * tp_fp64_exp(h.beta * l1p) * damp * tp_fp64_rcp(1 + plin * h.alpha);
+    // (a given P(k) may be negative: the library's log1p keeps its NaN below -1 and its infinity at -1)
+    const double grow = C.tab.nk ? exp(h.beta * log1p(plin)) : tp_fp64_exp(h.beta * tp_fp64_log1p(plin));
+    const double pq = plin * grow * damp * tp_fp64_rcp(1 + plin * h.alpha);
     return 2 * tpd::kPi * tpd::kPi * (pq + ph) * tp_fp64_rcp(k * k * k);
 }
 
 template <class T>
 __host__ __device__ T tp_halofit_k(const TpCosmoConst &C, T D1, T rs, T lrs, const TpHaloZT<T> &h, T k, T lk)
 {
-    if constexpr (std::is_same<T, double>::value) return tp_halofit_k64(C, D1, rs, lrs, h, k, lk);
+    if constexpr (std::is_same<T, double>::value)
+        if (tp_k_ordinary(lk)) return tp_halofit_k64(C, D1, rs, lrs, h, k, lk);
     const double twopi2 = 2 * tpd::kPi * tpd::kPi;
     const T plin = tp_pk_lin_log<T>(C, k, lk) * D1 * D1 * k * k * k / twopi2;
     const T y = k * rs, ly = lk + lrs, ysqr = y * y;
@@ -193,13 +199,17 @@ __host__ __device__ __forceinline__ T tp_pk_at(const TpCosmoConst &C, const TpZA
 
 // The ratio fitted to the T17 simulations, cuda_version/bispectrum.cu:971-979.
 // (1 + c1 k^-a1)^a1 / (1 + c2 k^-a2)^a3 evaluated as exp(a1 ln(1 + c1 e^(-a1 ln k)) - a3 ln(1 + c2 e^(-a2 ln k))).
+__host__ __device__ __forceinline__ double tp_t17_factor64(double lk)
+{
+    const double c1 = 9.5171e-4, c2 = 5.1543e-3, a1 = 1.3063, a2 = 1.1475, a3 = 0.62793;
+    return tp_fp64_exp(a1 * tp_fp64_log1p(c1 * tp_fp64_exp(-a1 * lk)) - a3 * tp_fp64_log1p(c2 * tp_fp64_exp(-a2 * lk)));
+}
 template <class T>
 __host__ __device__ __forceinline__ T tp_t17_factor(T lk)
 {
     const double c1 = 9.5171e-4, c2 = 5.1543e-3, a1 = 1.3063, a2 = 1.1475, a3 = 0.62793;
     if constexpr (std::is_same<T, double>::value)
-        return tp_fp64_exp(a1 * tp_fp64_log1p(c1 * tp_fp64_exp(-a1 * lk)) -
-                           a3 * tp_fp64_log1p(c2 * tp_fp64_exp(-a2 * lk)));
+        if (tp_k_ordinary(lk)) return tp_t17_factor64(lk);
     return exp(a1 * log1p(c1 * exp(-1. * a1 * lk)) - a3 * log1p(c2 * exp(-1. * a2 * lk)));
 }
 
@@ -346,17 +356,25 @@ __device__ __forceinline__ float tp_limber_pk_node32(const TpPNode32 &N, float e
 // are all of T1's work and are bound by FP64 issue, so a node takes the fewest instructions its factors allow: the
 // node's constants folded, the quotients merged, the damping in the exponent of (1 + Delta^2)^beta, and 1 / k^3 in
 // that of the T17 factor, whose logarithms need no more than their absolute rounding.  A T1 covariance of 210 pairs,
-// one MI355X: 155 ms with the library's functions, 81 with those of tp_fp64.h, 73-75 in this form, 64 with the logarithm's
-// table.
+// one MI355X: 155 ms with the library's functions, 81 with those of tp_fp64.h, 73-75 in this form, 64-66 with the logarithm's
+// table, 62 without ANY.
+// ANY: with the branch for a k outside tp_k_ordinary; without it, for callers that bound ell: the branch's library
+// functions fill the registers (T1: 128 and 352 bytes of spill, 72 ms, against 159 without spill, 62 ms).
+template <bool ANY = true>
 __host__ __device__ __forceinline__ double tp_limber_pk_node(const TpCosmoConst &C, const TpPNode &N, double ell,
                                                              double lell, int flags)
 {
     if (N.zero) return 0.0;
     const double k = ell * N.ifK, lk = lell - N.lfK;
+    if (ANY && !tp_k_ordinary(lk)) {
+        const double P = (flags & TP_PK_LINEAR) ? N.D1 * N.D1 * tp_pk_lin_log<double>(C, k, lk)
+                                                : tp_halofit_k<double>(C, N.D1, N.rs, N.lrs, N.h, k, lk);
+        return (flags & TP_PK_T17) ? tp_t17_factor<double>(lk) * N.pref * P : N.pref * P;
+    }
     if (C.tab.nk) {  // a given P(k)
         const double P = (flags & TP_PK_LINEAR) ? N.D1 * N.D1 * tp_pk_table(C.tab, k)
                                                 : tp_halofit_k64(C, N.D1, N.rs, N.lrs, N.h, k, lk);
-        return (flags & TP_PK_T17) ? tp_t17_factor<double>(lk) * N.pref * P : N.pref * P;
+        return (flags & TP_PK_T17) ? tp_t17_factor64(lk) * N.pref * P : N.pref * P;
     }
     double P = tp_fp64_exp(fma(N.ns3, lk, N.ld)) * tp_eh_r2(C, k * C.h);  // Delta^2
     if (!(flags & TP_PK_LINEAR)) {  // tp_halofit_k64 without its 2 pi^2 / k^3
