@@ -475,7 +475,9 @@ def test_point_calls_agree_at_every_size(fid_tables, mode, n):
 
 @pytest.mark.parametrize("n", [5, 70000, 140000])
 def test_non_finite_point_is_refused_and_leaves_no_flag(fid_tables, n):
-    """A non-finite ell ends the call with TP_ENONFINITE at any size, and the next call starts clean."""
+    """A non-finite ell ends the call with TP_ENONFINITE at any size, and the next call starts clean.  The flag word is
+    read when a value is not finite, so what shows it cleared is a call with such a value and no flag: a radius of 1e200
+    takes the filter to infinity times zero, where ell and B_kappa are finite, and that is returned, not refused."""
     x = np.tile([100.0, 200.0, 1.0], (n, 1))
     th = W.to_rad([2.0, 4.0, 8.0])
     bad = x.copy()
@@ -484,6 +486,7 @@ def test_non_finite_point_is_refused_and_leaves_no_flag(fid_tables, n):
     for call in (lambda: fid_tables.map3_integrand(bad, th), lambda: fid_tables.bkappa(bad)):
         with pytest.raises(tp.TpError, match="non-finite"):
             call()
+        assert np.all(np.isnan(fid_tables.map3_integrand(x, [1e200, 1e200, 1e200])))
         assert np.array_equal(fid_tables.map3_integrand(x, th), good)
 
 

@@ -281,8 +281,9 @@ static int check_cosmo(tp_ctx *ctx, const tp_cosmo *c, int icosmo)
 //     between two streams so that one's copy in and first waves fill the other's last (10^6 B_kappa points FP64:
 //     4.84 -> 2.72 ms).  The second stream is the batched engine's first: a stream of its own would share a hardware
 //     queue (there are four) with one of the engine's two and serialise their rounds (a 29.2 ms batch took 30.8).
-//   * The kernels' flag word stays zero between calls (cleared again when a call found it raised), and a raised flag
-//     always leaves a non-finite value behind, so it is read only when there is one.
+//   * The kernels' flag word is zero between calls: a call that found it raised, or that ends on an error, clears it and
+//     waits for that, since the next call's second stream is not ordered behind the clear.  A raised flag always leaves
+//     a non-finite value behind, so it is read only when there is one.
 constexpr size_t kPointsZeroCopyIn = 32768, kPointsChunk = 65536;
 
 template <class Launch>
@@ -299,10 +300,16 @@ static int run_points(tp_ctx *ctx, size_t npts, const double *in, double *out, L
     const size_t step = ((npts + nch - 1) / nch + 63) / 64 * 64;  // whole waves
     double *hin = (double *)ctx->h_in.p, *hout = (double *)ctx->h_out.p;
     int *d_flag = (int *)ctx->d_ptflag.p;
+    auto clear_flag = [&] {
+        hipLaunchKernelGGL(k_clear_word, dim3(1), dim3(1), 0, ctx->stream, d_flag);
+        const hipError_t e = hipGetLastError(), w = hipStreamSynchronize(ctx->stream);
+        return e != hipSuccess ? e : w;
+    };
     // on an error, let queued work drain before the buffers can be reused
     auto fail = [&](int e) {
         (void)hipStreamSynchronize(ctx->stream);
         if (nch > 1) (void)hipStreamSynchronize(ctx->lane[0].stream);
+        (void)clear_flag();
         return e;
     };
 #define TPP(call)                                                                                          \
@@ -341,8 +348,7 @@ static int run_points(tp_ctx *ctx, size_t npts, const double *in, double *out, L
     TPP(hipStreamSynchronize(ctx->stream));
     std::memcpy(&flag, ctx->h_out.p, sizeof(int));
     if (!flag) return 0;
-    hipLaunchKernelGGL(k_clear_word, dim3(1), dim3(1), 0, ctx->stream, d_flag);
-    TPP(hipGetLastError());
+    TPP(clear_flag());
 #undef TPP
     return tp_set_error(TP_ENONFINITE, std::string(what) + ": non-finite ell or B_kappa value");
 }
