@@ -142,7 +142,8 @@ int tp_map3_batch(tp_ctx *ctx, const tp_cosmo *c, size_t ntriples, const int *ic
  * workgroup, which evaluates the one-wavenumber terms of BiHalofit once per distinct multipole of
  * a region (47 per 33 points) in LDS.  By default the shape is tuned per launch-size bucket on the
  * first batched call of a context and precision (all shapes give bit-identical results).
- * lanes = 0 restores tuning; 1, 2, 4, 8, 16, 32 or 64 forces that shape.  No counterpart in the
+ * Rounds of up to 32 regions take one thread per (point, z-node) instead of the tuned shape.
+ * lanes = 0 restores this choice; 1, 2, 4, 8, 16, 32 or 64 forces that shape for every round.  No counterpart in the
  * reference (its GPU build has one fixed launch shape). */
 int tp_set_region_lanes(tp_ctx *ctx, int lanes);
 /* The tuned shapes of mode (TP_MODE_FP64 or TP_MODE_FP32) for launches of < 32k, < 160k,

@@ -197,6 +197,32 @@ def test_launch_shapes_bit_identical(gpu_ctx, fid_tables):
     assert all(x in (1, 2, 4, 8, 16, 32, 64) for x in tab)
 
 
+@pytest.mark.parametrize("mode", [tp.MODE_FP64, tp.MODE_FP32])
+@pytest.mark.parametrize("n", [1, 3, 40])
+def test_smallest_rounds_bit_identical(gpu_ctx, fid_nz, mode, n):
+    """Rounds of up to 32 regions take one thread per (point, node) unless a shape is forced, two points to a workgroup:
+    with 33 points to a region, every other region shares one with the next, here of another integral and cosmology.  Same
+    bits as the forced shapes."""
+    cosmos = [W.fiducial(), tp.Cosmology(om=0.25, sigma8=0.9, ns=0.95), tp.Cosmology(om=0.4, w=-0.8)]
+    tabs = tp.CosmologyTables(cosmos, fid_nz, 100, 3.0, gpu_ctx)
+    th = np.resize(W.to_rad(W.triples(W.map3_c0_radii())), (n, 3))
+    ic = np.arange(n) // 2 % 3  # the batch's two groups take every other integral: each has all cosmologies
+    gpu_ctx.set_round_log(True)
+    try:
+        a = tabs.map3_batch(th, ic, 1e-4, mode)
+        regions = gpu_ctx.round_log()[:, 1]
+        print("rounds of up to 32 regions: %d of %d" % ((regions <= 32).sum(), regions.size))
+        assert (regions <= 32).sum() >= (2 if n > 1 else 1)
+        for lanes in (1, 8, 16):
+            tp._check(tp.lib().tp_set_region_lanes(gpu_ctx.h, lanes), "tp_set_region_lanes")
+            b = tabs.map3_batch(th, ic, 1e-4, mode)
+            for x, y in zip(a, b):
+                assert np.array_equal(x, y), lanes
+    finally:
+        tp._check(tp.lib().tp_set_region_lanes(gpu_ctx.h, 0), "tp_set_region_lanes")
+        gpu_ctx.set_round_log(False)
+
+
 def test_given_pk_matches_oracle(gpu_ctx, fid_nz):
     """Tables, B_kappa and <Map^3> from a given linear P(k) (the cosmosis input,
     classed_version/bispectrum.cpp:81-89, 785-806) against the oracle's Pk_given branch."""
@@ -452,8 +478,10 @@ def test_map3_c1_all_triples_match_oracle_fixture(fid_tables):
     assert r32.max() < 1e-3
 
 
+# A call has at most 16 chunks: from 16 x 131072 points on they take the two-wave kernel, here with an odd number of waves' points
+# in each chunk and a part of one in the last
 @pytest.mark.parametrize("mode", [tp.MODE_FP64, tp.MODE_FP32, tp.MODE_ANALYTIC])
-@pytest.mark.parametrize("n", [1, 3, 4096, 4097, 32768, 32833, 131072, 200003])
+@pytest.mark.parametrize("n", [1, 3, 4096, 4097, 32768, 32833, 131072, 200003, 16 * 131136 - 50])
 def test_point_calls_agree_at_every_size(fid_tables, mode, n):
     """The evaluation calls split a point's nodes by the launch's size (one thread per node, 8 or 2 waves per point)
     and a large call into overlapping chunks; the summation tree is the same, so a point's value is the same bits in
@@ -465,7 +493,7 @@ def test_point_calls_agree_at_every_size(fid_tables, mode, n):
     ell[n // 2, 1] = 0.0
     x = np.column_stack([l, phi])
     th = W.to_rad([2.0, 4.0, 8.0])
-    few = np.unique(np.concatenate([[0, n // 2, n - 1], rng.integers(0, n, 200)]))
+    few = np.unique(np.concatenate([[0, n // 2, n - 1], n - 1 - np.arange(min(n, 130)), rng.integers(0, n, 200)]))
     b, f = fid_tables.bkappa(ell, 0, mode), fid_tables.map3_integrand(x, th, 0, mode)
     assert np.array_equal(b[few], fid_tables.bkappa(ell[few], 0, mode))
     assert np.array_equal(f[few], fid_tables.map3_integrand(x[few], th, 0, mode))

@@ -431,13 +431,15 @@ int grid_for(size_t n, int block) { return (int)((n + block - 1) / block); }
 
 }  // namespace
 
-// The split of a point's nodes by launch size, from whole calls of B_kappa (us; FP64, FP32 in brackets) with one
+// The split of a point's nodes by launch size, from calls of B_kappa in one launch (us; FP64, FP32 in brackets) with one
 // thread per (point, node), 8, 2 and 1 waves per point:
 //      33 points:  21 (20)   65 (35)  133 (57)  249 (95)     4 096:  45 (36)    68 (38)  136 (62)  254 (102)
 //     8 192:       90 (68)   93 (61)  160 (84)  278 (126)   32 768: 224 (159)  170 (107) 195 (116) 307 (156)
 //    65 536:                299 (174) 310 (183) 357 (204)  131 072:            555 (326) 546 (322) 576 (335)
 // one thread per (point, node) while its repeated set-up costs less than the shorter chain gains, 8 waves until the
-// launch fills the chip with fewer, then 2.
+// launch fills the chip with fewer, then 2.  A call is cut into launches of ~65 536 points, at most 16 of them, so the
+// last line is crossed by calls of 2.1 million points and more: 4 194 304 points in 16 launches 10.9 ms FP64 with 8 waves,
+// 10.6 with 2 (FP32 6.15 and 6.15); 8 388 608: 21.6 and 20.8 (12.4 and 12.2).
 constexpr size_t kNodePoints = 4096, kWidePoints = 131072;
 
 template <class T, bool MAP3>
