@@ -1,5 +1,5 @@
 """The FP64 exp, log and reciprocal of the z-node arithmetic (threepoint_amd/csrc/tp_fp64.h), built by the host
-compiler, against 80-bit arithmetic.  The bounds follow from the forms: exp is a degree-11 polynomial whose last
+compiler and (gpu) in a kernel, against 80-bit arithmetic.  The bounds follow from the forms: exp is a degree-11 polynomial whose last
 step rounds once at 0.5 ulp over an argument reduction good to 2^-56 and inner steps weighted by |r| < 0.35
 (< 1 ulp together); the reciprocal's third-order step leaves its cubed seed error and one rounding (< 1 ulp); exp10 is
 exp and the rounding of its remainder's product (< 1.5 ulp).  log ends in one rounded addition (0.5 ulp), and what is added to the exact
@@ -61,8 +61,7 @@ def _ulps(y, ref, absolute=0.0):
     return np.max(np.maximum(np.abs(y.astype(np.longdouble) - ref) - absolute, 0) / np.spacing(r))
 
 
-@pytest.mark.parametrize("what, bound", [(0, 1.0), (1, 0.51), (2, 1.0), (3, 1.01), (4, 1.5)])
-def test_errors(fp64, what, bound):
+def _samples(what):
     rng = np.random.default_rng(11 + what)
     if what == 0:  # every scale down to 0, and the whole range of normal results
         x = np.concatenate([rng.uniform(-700, 700, 200000), rng.uniform(-40, 40, 200000),
@@ -80,6 +79,15 @@ def test_errors(fp64, what, bound):
         x = np.concatenate([np.exp(rng.uniform(-100, 100, 400000)), rng.uniform(0, 3, 100000), [0.0, 1.0, 1e-300]])
     else:
         x = np.concatenate([rng.uniform(-300, 300, 200000), rng.uniform(-8, 8, 200000), np.arange(-300.0, 301.0)])
+    return x
+
+
+FORMS = [(0, 1.0), (1, 0.51), (2, 1.0), (3, 1.01), (4, 1.5)]
+
+
+@pytest.mark.parametrize("what, bound", FORMS)
+def test_errors(fp64, what, bound):
+    x = _samples(what)
     y, ref = fp64(what, x)
     u = _ulps(y, ref, 2.0 ** -60 if what in (1, 3) else 0.0)
     print("what %d: max error %.3f ulp of %d" % (what, u, x.size))
@@ -109,3 +117,38 @@ def test_the_whole_stated_domain_and_the_forms_for_any_argument(fp64):
         assert np.array_equal(fp64(form, x)[0], fp64(plain, x)[0])
     e = np.exp(np.random.default_rng(4).uniform(-700, 700, 20000))
     assert np.array_equal(fp64(7, e)[0], fp64(2, e)[0])
+
+
+def _device(what, x):
+    import ctypes
+    lib = ctypes.CDLL(os.path.join(ROOT, "tests", "fp64_device", "_build", "fp64_device.so"))
+    x = np.ascontiguousarray(x, dtype=np.float64)
+    y = np.zeros(x.size)
+    assert lib.run(what, x.size, x.ctypes.data_as(ctypes.c_void_p), y.ctypes.data_as(ctypes.c_void_p)) == 0
+    return y
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("what, bound", FORMS)
+def test_errors_on_the_device(what, bound):
+    """The forms as a kernel contains them, on the samples and to the bounds of the host build."""
+    x = _samples(what)
+    v = x.astype(np.longdouble)
+    ref = [np.exp, np.log, lambda t: 1 / t, np.log1p, lambda t: np.longdouble(10) ** t][what](v)
+    u = _ulps(_device(what, x), ref, 2.0 ** -60 if what in (1, 3) else 0.0)
+    print("what %d: max error %.3f ulp of %d" % (what, u, x.size))
+    assert u < bound
+
+
+@pytest.mark.gpu
+def test_ends_of_the_range_on_the_device():
+    """The range's ends and the forms for any argument, as in the host build."""
+    y = _device(0, [800.0, 2.0 ** 30, -800.0, -2.0 ** 30, 0.0, np.nan])
+    assert np.all(np.isposinf(y[:2])) and np.all(y[2:4] == 0) and y[4] == 1 and np.isnan(y[5])
+    far = np.array([1.5e9, 2.0 ** 31 - 1, 2.1e9, 1e15, 1e100, 1e300, np.inf])
+    assert np.all(np.isposinf(_device(5, far))) and np.all(_device(5, -far) == 0) and np.all(_device(6, -far) == 0)
+    y = _device(7, [np.inf, -np.inf, np.nan, 1.0, -4.0])
+    assert y[0] == 0 and not np.signbit(y[0]) and y[1] == 0 and np.signbit(y[1]) and np.isnan(y[2])
+    assert y[3] == 1 and y[4] == -0.25
+    x = _samples(2)
+    assert np.array_equal(_device(7, x), _device(2, x))

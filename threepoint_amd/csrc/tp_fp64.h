@@ -11,8 +11,8 @@
 // like the library's; a NaN stays a NaN; beyond 2^31 ln 2 = 1.49e9 the exponent's word wraps), exp10 up to 2^28, log any
 // positive normal one (a zero, a denormal, an infinity or a NaN gives some finite number: where one can arrive, another
 // factor of the same value carries it on), rcp any normal number whose reciprocal is normal.  The forms named _any and
-// _low take what these leave out, for the places it can reach.  Errors against 80-bit arithmetic, in a host build: exp
-// 0.91 ulp, exp10 1.19, rcp 0.50, log 0.50 ulp + 2^-60
+// _low take what these leave out, for the places it can reach.  Errors against 80-bit arithmetic, on the device and in a
+// host build alike: exp 0.91 ulp, exp10 1.19, rcp 0.50, log 0.50 ulp + 2^-60
 // (tests/test_fp64_math.py).  The logarithm's table is there because its other form, 2 atanh((m - 1) / (m + 1)) with a
 // reciprocal and a degree-15 series, takes 31 instructions to these 15 (25 issues to 18).
 //
@@ -80,13 +80,13 @@ __host__ __device__ __forceinline__ double tp_fp64_exp(double x)
 __host__ __device__ __forceinline__ double tp_fp64_exp_low(double x) { return tp_fp64_exp(__builtin_fmax(x, -0x1p30)); }
 __host__ __device__ __forceinline__ double tp_fp64_exp_any(double x) { return tp_fp64_exp_low(__builtin_fmin(x, 0x1p30)); }
 
-// hardware reciprocal (2^-27 or better) and one third-order step: error e^3 + the last rounding
+// hardware reciprocal (specified to 2^29 ulp: 2^-24) and one third-order step: error e^3 = 2^-72 and the last rounding
 __host__ __device__ __forceinline__ double tp_fp64_rcp_seed(double x)
 {
 #ifdef TP_FP64_DEVICE
     return __builtin_amdgcn_rcp(x);
 #else
-    return (1.0 / x) * (1.0 + 0x1p-27);  // an approximation of no more than the hardware's accuracy
+    return (1.0 / x) * (1.0 + 0x1p-24);  // an approximation of no more than the specified accuracy
 #endif
 }
 __host__ __device__ __forceinline__ double tp_fp64_rcp(double x)
