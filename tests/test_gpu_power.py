@@ -153,8 +153,8 @@ def test_map2_batch_sizes_agree(fid_tables, n, flags, sigma, reltol):
 
 @pytest.mark.parametrize("reltol", [5e-6, 5e-5])
 def test_map2_integrals_that_outgrow_the_device(gpu_ctx, fid_nz, reltol):
-    """A coarsely tabulated P(k) has kinks: integrals that hold more regions than the device keeps of one (all of
-    them at the tighter tolerance) are finished in rounds, with the bits of calls in rounds; a round limit ends the
+    """A coarsely tabulated P(k) has kinks: integrals that would hold more regions than the device keeps of one (all of
+    them at the tighter tolerance) are evaluated in rounds, with the bits of smaller calls; a round limit ends the
     call."""
     kh = np.geomspace(1e-4, 50, 12)
     tabs = tp.CosmologyTables([W.fiducial()], fid_nz, 100, 3.0, gpu_ctx, pk=(kh, 2e4 * (kh / 0.02) / (1 + (kh / 0.02) ** 2.5)))
@@ -172,6 +172,28 @@ def test_map2_integrals_that_outgrow_the_device(gpu_ctx, fid_nz, reltol):
             tabs.map2_batch(th, reltol=1e-5)
     finally:
         gpu_ctx.set_batch_limits()
+
+
+def test_map2_of_tabulated_pk_takes_the_device_where_it_fits(gpu_ctx, fid_nz):
+    """A table fine enough for the tolerance takes the device (one launch), a coarse one rounds, unless the tolerance is
+    loose.  A fine table that is rough from entry to entry is taken for smooth: integrals that then hold more regions than
+    the device keeps of one are finished in rounds.  The bits of calls in rounds (fewer than 16 integrals) each time."""
+    th = np.geomspace(0.5, 64, 28) * A
+    seen = set()
+    for nk, rough, reltol, device in [(500, 0.0, 1e-4, True), (150, 0.0, 1e-4, False), (12, 0.0, 1e-3, True),
+                                      (1000, 0.0, 3e-5, False), (1000, 0.02, 1e-4, True)]:
+        kh = np.geomspace(1e-4, 50, nk)
+        pk = 2e4 * (kh / 0.02) / (1 + (kh / 0.02) ** 2.5) * (1 + rough * (-1.0) ** np.arange(nk))
+        tabs = tp.CosmologyTables([W.fiducial()], fid_nz, 100, 3.0, gpu_ctx, pk=(kh, pk))
+        v, e, m = tabs.map2_batch(th, reltol=reltol)
+        launches, outgrown = gpu_ctx.stats()["launches"], int(((m // 17 + 1) // 2 > 1024).sum())
+        print("%d entries, %g: %d launches, %d of 28 outgrown" % (nk, reltol, launches, outgrown))
+        assert (launches == 1) == (device and not outgrown)
+        seen.add((device, outgrown > 0))
+        for c in (slice(0, 14), slice(14, 28)):
+            rv, re, rm = tabs.map2_batch(th[c], reltol=reltol)
+            assert np.array_equal(v[c], rv) and np.array_equal(e[c], re) and np.array_equal(m[c], rm)
+    assert {(True, False), (True, True)} <= seen
 
 
 def test_power_rejects_bad_arguments(fid_tables):

@@ -100,6 +100,7 @@ struct tp_cosmo {
     void *d_pnode = nullptr;          // [ncosmo][96] TpPNode: the P Limber sum's z-nodes (tp_power.hip)
     void *d_pnode32 = nullptr;        // [ncosmo][96] TpPNode32: their FP32 form (same allocation)
     int pk_nk = 0;                    // 0: Eisenstein & Hu
+    double pk_dlnk = 0;               // largest step in ln k of any cosmology's tabulated P(k)
     std::vector<TpCosmoConst> h_const;
 };
 

@@ -1098,17 +1098,27 @@ int map2_regions(tp_ctx *ctx, const tp_cosmo *c, const std::vector<TpPowerDesc> 
 // integrals the chip is empty either way and the host's heaps are faster than thread 0's (1 integral 0.9 ms in rounds,
 // 1.4 on the device; 8: 1.4-1.75 and 1.6; 16: 2.0 and 1.65).  Below kMap2Reltol integrals outgrow kMap2Regions (held at
 // most: 690 regions at 1e-5, 1250 at 3e-6, 2030 at 1e-6), so that their work there is lost (40 integrals, 1e-7: 5-6 ms in
-// rounds, 12 with the device first).
+// rounds, 12 with the device first).  A tabulated P(k) has a kink at each entry, of the size of its interpolation error,
+// dlnk^2 / 8 of P: below that, integrals outgrow the device from looser tolerances on (300 integrals at 1e-4, 150 entries
+// over 13 e-folds: 7-10 ms in rounds, 10-13 with the device first; 500 entries: 2.8-4.6 and 0.5-1.6).  They go there when
+// the tolerance is above that error and above kMap2TabReltol (at 3e-5, 1000 entries with acoustic oscillations: even), or
+// above kMap2TabLoose, where no table made them outgrow (1.6-6 ms in rounds, 0.6-1.5).
 constexpr size_t kMap2Few = 16;
-constexpr double kMap2Reltol = 5e-6;
+constexpr double kMap2Reltol = 5e-6, kMap2TabReltol = 5e-5, kMap2TabLoose = 1e-3;
 constexpr int kMap2Slice = 65536;
+bool map2_on_device(const tp_cosmo *c, size_t n, double reltol)
+{
+    if (n < kMap2Few) return false;
+    if (!c->pk_nk) return reltol >= kMap2Reltol;
+    return reltol >= kMap2TabLoose || (reltol >= kMap2TabReltol && reltol >= c->pk_dlnk * c->pk_dlnk / 8);
+}
 int map2_integrals(tp_ctx *ctx, const tp_cosmo *c, const std::vector<TpPowerDesc> &desc, const double *lo,
                    const double *hi, double reltol, double *out, double *err, long long *neval)
 {
     using clk = std::chrono::steady_clock;
     const auto t0 = clk::now();
     const size_t n = desc.size();
-    if (n < kMap2Few || !(reltol >= kMap2Reltol)) return map2_regions(ctx, c, desc, lo, hi, reltol, out, err, neval);
+    if (!map2_on_device(c, n, reltol)) return map2_regions(ctx, c, desc, lo, hi, reltol, out, err, neval);
     tp_batch_stats st{};
     int rc, ncu = 0;
     TP_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, ctx->device));
