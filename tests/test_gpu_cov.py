@@ -47,6 +47,18 @@ def test_t1_of_far_multipoles(fid_tables, fid_oracle):
     assert m[0] == n[1] and w[0] == v[1]
 
 
+def test_t2_of_far_multipoles(fid_tables, fid_oracle):
+    """The same for T2 of a finite survey (as small as the far radii, so that its window does not oscillate below them): a
+    batch with a far pair takes the point kernel with the branch."""
+    far, near, tx = np.full(6, 1e-16), np.array([6, 6, 12, 4, 8, 16], dtype=float) * A, 1e-15
+    args = (tp.GEOMETRY_CIRCLE, tx, 0.0, 0.0, 0.0, NGAL, 0)
+    v, n = fid_tables.map3_cov_t2(np.array([far, near]), *args, reltol=1e-3)
+    ov, on = fid_oracle.t2_total(far[:3], far[3:], 0, tx, 0.0, 0.0, 0.0, NGAL, 0, 1e-3)
+    assert n[0] == on and abs(v[0] / ov - 1) < 1e-10
+    w, m = fid_tables.map3_cov_t2(near[None, :], *args, reltol=1e-3)
+    assert m[0] == n[1] and w[0] == v[1]
+
+
 def test_t1_shape_noise_closed_form_on_gpu(fid_tables):
     th = np.array([3.0, 6.0, 12.0]) * A
     pairs = np.repeat(th[:, None], 6, axis=1)

@@ -64,6 +64,13 @@ __device__ __forceinline__ double uhat(double eta)
     return t * exp(-t);
 }
 
+// The covariance integrals take their Pell without the branch for far wavenumbers (tp_limber_pk_node<false>) when their
+// domains end below this: k = ell / f_K then stays below 3e19 h/Mpc (f_K > 0.03 Mpc/h from the first z that counts on, and
+// ell is a sum of up to three components), and, ell being made of the rule points of bisected domains, above the 1e-70 at
+// which the short forms would underflow.  With the branch in every kernel T1 took 72 ms for 65, and the finite-survey
+// T1's points with a tabulated P(k) 148 for 86.
+constexpr double kOrdinaryEll = 1e15;
+
 // Pell from the z-node records N[96] (pairs 2j, 2j+1 at cx -+ dx x_j): the cuda_version's device Pell
 // (bispectrum.cu:511-529), node pairs added in the reference's order (GQ96_of_Pk, bispectrum.cpp:1034-1046).
 template <bool ANY = true>
@@ -154,6 +161,7 @@ __device__ __forceinline__ double sinc_cut(double t) { return fabs(t) <= 1e-6 ? 
 // The T2 integrands at one point (apertureStatisticsCovariance.cu:2014-2110), in the reference's
 // product order: kT2A integrand_T2_part1 (ell Pell uHat uHat), kT2Circle integrand_T2_part2_circle,
 // kT2Square / kT2Rect integrand_T2_part2_square / _rectangle over (ell_x, ell_y).
+template <bool ANY>
 __device__ double t2_point(const TpCosmoConst &C, const TpPNode *__restrict__ N, const TpPowerDesc &D,
                            const double *x, double dx)
 {
@@ -163,12 +171,12 @@ __device__ double t2_point(const TpCosmoConst &C, const TpPNode *__restrict__ N,
         const double ell = x[0];
         if (ell < D.lmin) return 0;
         if (D.kind == kT2A) {
-            double r = ell * pell_nodes(C, N, ell, D.flags, dx, shot);
+            double r = ell * pell_nodes<ANY>(C, N, ell, D.flags, dx, shot);
             r *= uhat(ell * D.th[0]) * uhat(ell * D.th[1]);
             return r;
         }
         const double G = g_circle(ell, D.th[2]);
-        double r = pell_nodes(C, N, ell, D.flags, dx, shot);
+        double r = pell_nodes<ANY>(C, N, ell, D.flags, dx, shot);
         r *= ell * uhat(ell * D.th[0]) * uhat(ell * D.th[1]);
         r *= G;
         return r;
@@ -178,7 +186,7 @@ __device__ double t2_point(const TpCosmoConst &C, const TpPNode *__restrict__ N,
     const double G = a * a * b * b;
     const double ell = sqrt(lx * lx + ly * ly);
     if (ell < D.lmin) return 0;
-    double r = pell_nodes(C, N, ell, D.flags, dx, shot);
+    double r = pell_nodes<ANY>(C, N, ell, D.flags, dx, shot);
     r *= uhat(ell * D.th[0]) * uhat(ell * D.th[1]);
     r *= G;
     return r;
@@ -188,6 +196,7 @@ __device__ double t2_point(const TpCosmoConst &C, const TpPNode *__restrict__ N,
 // the window's wave vector, (c, d) and (e, f) two of the Pell wave vectors, l1 = |(a - c - e, b - d - f)|;
 // the circle cuts l_i <= lMin, the square and the rectangle l_i <= 0 and l3 > lMax; the reference's
 // product order.
+template <bool ANY>
 __device__ double t1fin_point(const TpCosmoConst &C, const TpPNode *__restrict__ N, const TpPowerDesc &D,
                               const double *x, double dx)
 {
@@ -208,15 +217,17 @@ __device__ double t1fin_point(const TpCosmoConst &C, const TpPNode *__restrict__
         return 0;
     }
     const double shot = 0.5 * D.sigma * D.sigma / D.ngal;
-    double r = pell_nodes(C, N, ell1, D.flags, dx, shot) * pell_nodes(C, N, ell2, D.flags, dx, shot) *
-               pell_nodes(C, N, ell3, D.flags, dx, shot);
+    double r = pell_nodes<ANY>(C, N, ell1, D.flags, dx, shot) * pell_nodes<ANY>(C, N, ell2, D.flags, dx, shot) *
+               pell_nodes<ANY>(C, N, ell3, D.flags, dx, shot);
     r *= uhat(ell1 * D.th[0]) * uhat(ell2 * D.th[1]) * uhat(ell3 * D.th[2]);
     r *= uhat(ell1 * D.th[3]) * uhat(ell2 * D.th[4]) * uhat(ell3 * D.th[5]);
     r *= G;
     return r;
 }
 
-// One thread per point; pdesc[i] names the integral (desc entry) of point i.
+// One thread per point; pdesc[i] names the integral (desc entry) of point i.  ANY: the covariance kinds' multipoles may have
+// any size (the rule is kOrdinaryEll's; the other kinds look at each k).
+template <bool ANY>
 __global__ void k_power_points(const TpCosmoConst *__restrict__ cc, const double *__restrict__ tab, int n_z,
                                const TpPowerDesc *__restrict__ desc,
                                const int *__restrict__ pdesc, size_t npts, int dim, const double *__restrict__ x,
@@ -240,9 +251,9 @@ __global__ void k_power_points(const TpCosmoConst *__restrict__ cc, const double
         tp_z_at<double>(T, n_z, C.zmax, xi[1], &Z);
         v = tp_pk_at<double>(C, Z, xi[0], xi[1], D.flags);
     } else if (D.kind >= kT1Circle) {
-        v = t1fin_point(C, pnode + (size_t)D.icosmo * TP_NNODES, D, xi, dx);
+        v = t1fin_point<ANY>(C, pnode + (size_t)D.icosmo * TP_NNODES, D, xi, dx);
     } else if (D.kind >= kT2A) {
-        v = t2_point(C, pnode + (size_t)D.icosmo * TP_NNODES, D, xi, dx);
+        v = t2_point<ANY>(C, pnode + (size_t)D.icosmo * TP_NNODES, D, xi, dx);
     } else {
         v = covg_point(C, T, n_z, xi[0], xi[1], xi[2], xi[3], D.th);
     }
@@ -267,10 +278,7 @@ template <bool F32> struct T1Shape {
 };
 constexpr int kT1Pell = 14 + TP_NPTS_GM3;     // Pell per region
 
-// F32: the Pell from the FP32 node records (pell_nodes32); ANY: pell_nodes for multipoles of any size.  The rule: without
-// it up to kT1OrdinaryEll, where k = ell / f_K stays below 3e19 h/Mpc (f_K > 0.03 Mpc/h from the first z that counts on)
-// and, ell being a rule point of a bisected [lmin, lmax], above the 1e-70 at which the short forms would underflow.
-constexpr double kT1OrdinaryEll = 1e15;
+// F32: the Pell from the FP32 node records (pell_nodes32); ANY: pell_nodes for multipoles of any size (kOrdinaryEll)
 template <bool F32, bool ANY>
 __global__ void __launch_bounds__(T1Shape<F32>::block) k_t1_regions(const TpCosmoConst *__restrict__ cc,
                                                     const TpPNode *__restrict__ pnode,
@@ -708,7 +716,7 @@ int check_args(tp_ctx *ctx, const tp_cosmo *c, int flags)
 // Evaluates npts points x (dim doubles each) of the integrals desc (pdesc[i] per point, or all of
 // desc[0] when pdesc is null); fval receives npts values.  Synchronous.
 int power_launch(tp_ctx *ctx, const tp_cosmo *c, const std::vector<TpPowerDesc> &desc, const int *pdesc, size_t npts,
-                 int dim, const double *x, double *fval)
+                 int dim, const double *x, double *fval, bool any = false)
 {
     if (npts == 0) return 0;
     int rc;
@@ -727,7 +735,7 @@ int power_launch(tp_ctx *ctx, const tp_cosmo *c, const std::vector<TpPowerDesc> 
     TP_HIP(hipMemcpyAsync(ctx->d_desc.p, desc.data(), bd, hipMemcpyHostToDevice, ctx->stream));
     TP_HIP(hipEventRecord(ctx->ev0, ctx->stream));
     const unsigned blk = 256;
-    hipLaunchKernelGGL(k_power_points, dim3((unsigned)((npts + blk - 1) / blk)), dim3(blk), 0, ctx->stream,
+    hipLaunchKernelGGL(any ? k_power_points<true> : k_power_points<false>, dim3((unsigned)((npts + blk - 1) / blk)), dim3(blk), 0, ctx->stream,
                        c->d_const, c->d_tab, c->n_z, (const TpPowerDesc *)ctx->d_desc.p,
                        pdesc ? (const int *)ctx->d_misc.p : nullptr, npts, dim, (const double *)ctx->d_in.p,
                        (double *)ctx->d_out.p, (int *)ctx->d_flag.p, (const TpPNode *)c->d_pnode, c->z_max / 2);
@@ -761,6 +769,10 @@ int power_batch(tp_ctx *ctx, const tp_cosmo *c, const std::vector<TpPowerDesc> &
     for (size_t k = 0; k < nint; ++k)
         if (!I[k].init(D, 1, lo + D * k, hi + D * k, 0, 0, reltol, tpc::L1))
             return tp_set_error(TP_EINVAL, "bad integration domain");
+    bool any = false;  // covariance integrals with far multipoles
+    for (size_t k = 0; k < nint; ++k)
+        for (unsigned d = 0; d < D; ++d)
+            any |= desc[k].kind >= kT2A && !(std::fabs(lo[D * k + d]) <= kOrdinaryEll && std::fabs(hi[D * k + d]) <= kOrdinaryEll);
     const unsigned np = tpc::rule_points(D);
     std::vector<size_t> active(nint), offs;
     for (size_t k = 0; k < nint; ++k) active[k] = k;
@@ -797,7 +809,7 @@ int power_batch(tp_ctx *ctx, const tp_cosmo *c, const std::vector<TpPowerDesc> &
                     for (unsigned q = 0; q < np; ++q) pdesc[o + q] = (int)active[a];
                 }
             }
-            int rc = power_launch(ctx, c, desc, pdesc.data(), npts, (int)D, pts.data(), vals.data());
+            int rc = power_launch(ctx, c, desc, pdesc.data(), npts, (int)D, pts.data(), vals.data(), any);
             if (rc) return rc;
             ctx->stats.points += (long long)npts;
 #pragma omp parallel for schedule(dynamic, 16) num_threads(nt) if (a1 - a0 > 64)
@@ -1214,7 +1226,7 @@ int t1_regions(tp_ctx *ctx, const tp_cosmo *c, const std::vector<TpPowerDesc> &d
                const double *hi, double reltol, double area, int mode, double *out, long long *neval)
 {
     bool any = false;
-    for (const TpPowerDesc &D : desc) any |= !(D.lmax <= kT1OrdinaryEll);
+    for (const TpPowerDesc &D : desc) any |= !(D.lmax <= kOrdinaryEll);
     auto launch = [&](size_t nreg, const TpRegion *d_reg, TpRegionOut *d_out, double *, hipStream_t st,
                       hipEvent_t evm) -> int {
         const bool f32 = mode == TP_MODE_FP32;

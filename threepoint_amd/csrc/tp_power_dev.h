@@ -162,9 +162,9 @@ __host__ __device__ __forceinline__ double tp_halofit_k64(const TpCosmoConst &C,
     const double ph = h.a * tp_fp64_exp(h.f1 * 3 * ly) * ysqr * tp_fp64_rcp(den * (ysqr + h.xnu));
     // the damping's argument is the one that leaves the range of the short exp (y up to any ell rs / f_K)
     const double damp = tp_fp64_exp(fmax(-y * 0.25 - ysqr * 0.125, -1000.0));
-    // (a given P(k) may be negative: the library's log1p keeps its NaN below -1 and its infinity at -1)
-    const double grow = C.tab.nk ? exp(h.beta * log1p(plin)) : tp_fp64_exp(h.beta * tp_fp64_log1p(plin));
-    const double pq = plin * grow * damp * tp_fp64_rcp(1 + plin * h.alpha);
+    // (a given P(k) may be negative: the library's log1p keeps its NaN below -1)
+    const double l1p = C.tab.nk ? log1p(plin) : tp_fp64_log1p(plin);
+    const double pq = plin * tp_fp64_exp(h.beta * l1p) * damp * tp_fp64_rcp(1 + plin * h.alpha);
     return 2 * tpd::kPi * tpd::kPi * (pq + ph) * tp_fp64_rcp(k * k * k);
 }
 
@@ -357,9 +357,9 @@ __device__ __forceinline__ float tp_limber_pk_node32(const TpPNode32 &N, float e
 // node's constants folded, the quotients merged, the damping in the exponent of (1 + Delta^2)^beta, and 1 / k^3 in
 // that of the T17 factor, whose logarithms need no more than their absolute rounding.  A T1 covariance of 210 pairs,
 // one MI355X: 155 ms with the library's functions, 81 with those of tp_fp64.h, 73-75 in this form, 64-66 with the logarithm's
-// table, 62 without ANY.
+// table.
 // ANY: with the branch for a k outside tp_k_ordinary; without it, for callers that bound ell: the branch's library
-// functions fill the registers (T1: 128 and 352 bytes of spill, 72 ms, against 159 without spill, 62 ms).
+// functions fill the registers (T1: 128 and 352 bytes of spill, 72 ms, against 65).
 template <bool ANY = true>
 __host__ __device__ __forceinline__ double tp_limber_pk_node(const TpCosmoConst &C, const TpPNode &N, double ell,
                                                              double lell, int flags)
