@@ -39,7 +39,7 @@ PEAK = {"fp64": 78.6e12, "fp32": 157.3e12, "bf16": 2.5e15, "fp16": 2.5e15, "hbm"
 # WRITE_SIZE over benchMap3.x (profiles/map3_c3_counters.md), each counter scaled by its reading for
 # k_copy16 copying 1 GiB (FETCH_SIZE x2.000, WRITE_SIZE x1.000).  Algorithmic: 64/33 B of region in +
 # 8 B of integrand value out.
-HBM_BYTES_PER_POINT = {"double": 12.92, "float": 11.66}
+HBM_BYTES_PER_POINT = {"double": 15.40, "float": 24.85}
 # The surrogate network 8 -> 4 x 256 -> 1: algorithmic flops per point 2 (8 x 256 + 3 x 256 x 256 + 256); the
 # inference kernel k_mlp_h executes the three 256 x 256 layers as one FP16 MFMA per weight fragment and
 # layer 1 on the FP32 MFMA, i.e. the algorithmic MFMA work.
@@ -49,15 +49,15 @@ MLP_MFMA_FLOPS_EXECUTED = 2 * (8 * 256 + 3 * 256 * 256)
 # VALU flops = SQ_INSTS_VALU_FLOPS_* x 64, MFMA busy = SQ_VALU_MFMA_BUSY_CYCLES / (GRBM_GUI_ACTIVE / 8 XCDs
 # x 256 CUs x 4 SIMDs), each rate over the kernel's summed dispatch time in the counter run.
 MLP_HBM_BYTES_PER_POINT = 43.5
-MLP_COUNTERS = {"kernel": "k_mlp_h", "mfma_tflops": 877.8, "mfma_frac_of_fp16_peak": 0.351, "mfma_busy": 0.46,
-                "valu_fp32_tflops": 10.3, "hbm_read_bytes_per_point": 35.5, "hbm_write_bytes_per_point": 8.0}
+MLP_COUNTERS = {"kernel": "k_mlp_h", "mfma_tflops": 863.8, "mfma_frac_of_fp16_peak": 0.346, "mfma_busy": 0.46,
+                "valu_fp32_tflops": 10.1, "hbm_read_bytes_per_point": 35.5, "hbm_write_bytes_per_point": 8.0}
 REGION_COUNTERS = {
-    "float": {"kernel": "k_region_cached<float, 1>", "valu_fp32_tflops": 36.2, "frac_of_fp32_peak": 0.230,
-              "frac_of_scalar_fp32": 0.460, "valu_fp32_flops_per_point": 22240, "trans_fp32_per_point": 2720,
-              "hbm_read_bytes_per_point": 3.59, "hbm_write_bytes_per_point": 8.08},
-    "double": {"kernel": "k_region_cached<double, 1>", "valu_fp64_tflops": 39.5, "frac_of_fp64_peak": 0.502,
-               "valu_fp64_flops_per_point": 93400, "hbm_read_bytes_per_point": 4.85,
-               "hbm_write_bytes_per_point": 8.08},
+    "float": {"kernel": "k_region_cached<float, 1>", "valu_fp32_tflops": 44.1, "frac_of_fp32_peak": 0.280,
+              "frac_of_scalar_fp32": 0.561, "valu_fp32_flops_per_point": 19990, "trans_fp32_per_point": 2516,
+              "hbm_read_bytes_per_point": 5.19, "hbm_write_bytes_per_point": 19.66},
+    "double": {"kernel": "k_region_cached<double, 1>", "valu_fp64_tflops": 51.2, "frac_of_fp64_peak": 0.651,
+               "valu_fp64_flops_per_point": 69070, "hbm_read_bytes_per_point": 7.26,
+               "hbm_write_bytes_per_point": 8.14},
 }
 FLOPS_PER_ELEM = 20.0
 CENSUS_FILE = os.path.join("tests", "golden", "census.json")
