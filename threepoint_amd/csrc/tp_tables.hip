@@ -726,7 +726,7 @@ static int cosmo_build(tp_ctx *ctx, int ncosmo, const tp_cosmology *params, cons
     // tabulated P(k): strictly increasing positive k, finite P (the reference keeps a std::map)
     std::vector<double> hk, hp, hl0, hinv;
     std::vector<int> hidx;
-    double dlnk = 0;
+    double step = 1;  // largest k_j+1 / k_j
     const int ng = nk > 0 ? std::max(64, 4 * nk) : 0;
     if (nk) {
         if (nk < 2 || !pk_k || !pk_p) return tp_set_error(TP_EINVAL, "tp_cosmo_build_pk: need at least 2 P(k) entries");
@@ -741,7 +741,7 @@ static int cosmo_build(tp_ctx *ctx, int ncosmo, const tp_cosmology *params, cons
                 if (!(ks[j] > 0) || !std::isfinite(ks[j]) || !std::isfinite(ps[j]) || (j && !(ks[j] > ks[j - 1])))
                     return tp_set_error(TP_EINVAL, "tp_cosmo_build_pk: k must be positive and strictly increasing, "
                                                    "P finite (cosmology " + std::to_string(i) + ")");
-                if (j) dlnk = std::max(dlnk, std::log(ks[j] / ks[j - 1]));
+                if (j) step = std::max(step, ks[j] / ks[j - 1]);
                 hk[(size_t)i * nk + j] = ks[j];
                 hp[(size_t)i * nk + j] = ps[j];
             }
@@ -822,7 +822,7 @@ static int cosmo_build(tp_ctx *ctx, int ncosmo, const tp_cosmology *params, cons
         d_inv = d_l0 + ncosmo;
         d_idx = (int *)(d_inv + ncosmo);
         c->pk_nk = nk;
-        c->pk_dlnk = dlnk;
+        c->pk_dlnk = std::log(step);
         TPC(hipMemcpy(d_pkk, hk.data(), nkt * sizeof(double), hipMemcpyHostToDevice));
         TPC(hipMemcpy(d_pkp, hp.data(), nkt * sizeof(double), hipMemcpyHostToDevice));
         TPC(hipMemcpy(d_l0, hl0.data(), ncosmo * sizeof(double), hipMemcpyHostToDevice));
